@@ -51,6 +51,7 @@ struct pf_net {
     // gradients of activations
     bf16 *g5 = nullptr, *gu1 = nullptr, *g4 = nullptr, *gu2 = nullptr, *g3 = nullptr, *gp2 = nullptr, *gp1 = nullptr;
     float* fin = nullptr;  // fp32 staging of host inputs
+    float* part = nullptr; // partial weight gradients of one layer (training only)
     // dataset
     int max_samples = 0;
     bf16* dfeat = nullptr;
@@ -90,45 +91,60 @@ static int gridn(long long n, int threads = 256, int cap = 8192) {
 }
 
 // ---------------------------------------------------------------------------
-// convolution dispatch (CIN and the channel-group width are template arguments)
+// convolution dispatch
 // ---------------------------------------------------------------------------
+// Launch shape of k_conv3: output channels per block (16 NT) and x rows per wave (ZT x YT).
+// Larger blocks reuse weights and halo more; smaller ones give a small volume enough blocks
+// for the 256 CUs.
+static long long conv_blocks(const Vol& o, int ZT, int YT) {
+    return (long long)ceil_div(o.nx, 16) * ceil_div(o.ny, 2 * YT) * ceil_div(o.nz, 2 * ZT);
+}
+
+template <int CIN, int NT, int ZT, int YT, bool UP, bool RELU>
+static void conv_launch(pf_net* net, const Vol& o, const bf16* in, const bf16* w, const float* bias, const bf16* skip,
+                        bf16* out, int cout) {
+    hipLaunchKernelGGL((k_conv3<CIN, NT, ZT, YT, UP, RELU>), dim3((unsigned)conv_blocks(o, ZT, YT), cout / (16 * NT)),
+                       dim3(256), 0, net->stream, o, in, w, bias, skip, out, cout);
+}
+
 template <int CIN, bool UP, bool RELU>
-static void conv_cin(pf_net* net, const Vol& o, const bf16* in, const bf16* w, const float* bias, const bf16* skip,
-                     bf16* out, int cout) {
-    const long long tiles = o.n() / 16;
-    if (cout % 64 == 0) {
-        const long long waves = tiles * (cout / 64);
-        hipLaunchKernelGGL((k_conv3<CIN, 4, UP, RELU>), dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, net->stream, o,
-                           in, w, bias, skip, out, cout);
-    } else {
-        const long long waves = tiles * (cout / 32);
-        hipLaunchKernelGGL((k_conv3<CIN, 2, UP, RELU>), dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, net->stream, o,
-                           in, w, bias, skip, out, cout);
-    }
-}
-
-template <bool UP, bool RELU>
-static void conv(pf_net* net, const Vol& o, int cin, const bf16* in, const bf16* w, const float* bias, const bf16* skip,
+static void conv(pf_net* net, const Vol& o, const bf16* in, const bf16* w, const float* bias, const bf16* skip,
                  bf16* out, int cout) {
-    switch (cin) {
-        case 8: conv_cin<8, UP, RELU>(net, o, in, w, bias, skip, out, cout); break;
-        case 32: conv_cin<32, UP, RELU>(net, o, in, w, bias, skip, out, cout); break;
-        case 64: conv_cin<64, UP, RELU>(net, o, in, w, bias, skip, out, cout); break;
-        case 128: conv_cin<128, UP, RELU>(net, o, in, w, bias, skip, out, cout); break;
+    constexpr long long MINB = 512;  // blocks wanted (256: 2 % slower, 1024: 2 %)
+    const long long b24 = conv_blocks(o, 2, 4), b22 = conv_blocks(o, 2, 2);
+    const int n4 = cout / 64, n2 = cout / 32;
+    if (CIN >= 32 && n4 && b24 * n4 >= MINB) {
+        if constexpr (CIN >= 32) conv_launch<CIN, 4, 2, 4, UP, RELU>(net, o, in, w, bias, skip, out, cout);
+    } else if (b24 * n2 >= MINB) {
+        conv_launch<CIN, 2, 2, 4, UP, RELU>(net, o, in, w, bias, skip, out, cout);
+    } else if (UP || b22 * n2 >= MINB) {
+        conv_launch<CIN, 2, 2, 2, UP, RELU>(net, o, in, w, bias, skip, out, cout);
+    } else {
+        if constexpr (!UP) conv_launch<CIN, 2, 1, 1, UP, RELU>(net, o, in, w, bias, skip, out, cout);
     }
 }
 
-template <bool UP>
-static void wgrad(pf_net* net, const Vol& o, const bf16* gy, const bf16* x, float* gw, int cout, int cin) {
-    const int vchunk = 4096;
-    const long long nch = (o.n() + vchunk - 1) / vchunk;
-    const long long waves = 27LL * (cout / 16) * ((cin + 15) / 16) * nch;
-    hipLaunchKernelGGL((k_conv3_wgrad<UP>), dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, net->stream, o, gy, x, gw,
-                       cout, cin, vchunk);
+// Blocks over the voxels and slots of partial sums of one weight-gradient launch: about 256
+// blocks in all (one per CU: the accumulators take most of a wave's registers), each with
+// its own slot per wave that shares a channel tile.
+template <int CIN, bool UP> static int wgrad_chunks(const Vol& o, int cout) {
+    using G = WGrad<CIN, UP>;
+    const int bricks = ceil_div(o.nx, 16) * ceil_div(o.ny, 2 * G::YT) * ceil_div(o.nz, 4);
+    return std::max(1, std::min(bricks, 256 / ((cout / 32) * (CIN / G::CB))));
+}
+template <int CIN, bool UP> static size_t wgrad_part(const Vol& o, int cout) {
+    return (size_t)wgrad_chunks<CIN, UP>(o, cout) * WGrad<CIN, UP>::KS * ((size_t)27 * cout * CIN + cout);
 }
 
-static void chan_sum(pf_net* net, long long nv, int c, const bf16* g, float* gb) {
-    hipLaunchKernelGGL(k_chan_sum, dim3(gridn(nv * c, 256, 2048)), dim3(256), 0, net->stream, nv, c, g, gb);
+// gw, gb: the layer's weight and bias gradients (consecutive in the parameter vector)
+template <int CIN, bool UP>
+static void wgrad(pf_net* net, const Vol& o, const bf16* gy, const bf16* x, float* gw, int cout) {
+    using G = WGrad<CIN, UP>;
+    const int chunks = wgrad_chunks<CIN, UP>(o, cout), n = 27 * cout * CIN + cout;
+    hipLaunchKernelGGL((k_conv3_wgrad<CIN, UP>), dim3(chunks, (cout / 32) * (CIN / G::CB)), dim3(256), 0, net->stream,
+                       o, gy, x, net->part, cout);
+    hipLaunchKernelGGL(k_wgrad_reduce, dim3(ceil_div(n, 16)), dim3(256), 0, net->stream, chunks * G::KS, n,
+                       (const float*)net->part, gw);
 }
 
 static void prep_weights(pf_net* net) {
@@ -136,7 +152,7 @@ static void prep_weights(pf_net* net) {
         Layer& L = net->layer[l];
         const long long n = 27LL * L.cout * L.cin;
         hipLaunchKernelGGL(k_prep_weights, dim3(gridn(n)), dim3(256), 0, net->stream, net->p + L.w_off, L.cout, L.cin,
-                           L.cin, L.wf, L.wt);
+                           L.wf, L.wt);
     }
     net->weights_ready = true;
 }
@@ -147,13 +163,13 @@ static void forward(pf_net* net) {
     const Vol &V1 = net->L[0], &V2 = net->L[1], &V3 = net->L[2];
     Layer* Ly = net->layer;
     float* P = net->p;
-    conv<false, true>(net, V1, NIN, net->x, Ly[0].wf, P + Ly[0].b_off, nullptr, net->e1, 32);
-    hipLaunchKernelGGL(k_pool, dim3(gridn(V2.n() * 32)), dim3(256), 0, net->stream, V2, net->e1, net->p1, 32);
-    conv<false, true>(net, V2, 32, net->p1, Ly[1].wf, P + Ly[1].b_off, nullptr, net->e2, 64);
-    hipLaunchKernelGGL(k_pool, dim3(gridn(V3.n() * 64)), dim3(256), 0, net->stream, V3, net->e2, net->p2, 64);
-    conv<false, true>(net, V3, 64, net->p2, Ly[2].wf, P + Ly[2].b_off, nullptr, net->e3, 128);
-    conv<true, true>(net, V2, 128, net->e3, Ly[3].wf, P + Ly[3].b_off, net->e2, net->d2, 64);
-    conv<true, true>(net, V1, 64, net->d2, Ly[4].wf, P + Ly[4].b_off, net->e1, net->d1, 32);
+    conv<NIN, false, true>(net, V1, net->x, Ly[0].wf, P + Ly[0].b_off, nullptr, net->e1, 32);
+    hipLaunchKernelGGL(k_pool, dim3(gridn(V2.n() * 4)), dim3(256), 0, net->stream, V2, net->e1, net->p1, 32);
+    conv<32, false, true>(net, V2, net->p1, Ly[1].wf, P + Ly[1].b_off, nullptr, net->e2, 64);
+    hipLaunchKernelGGL(k_pool, dim3(gridn(V3.n() * 8)), dim3(256), 0, net->stream, V3, net->e2, net->p2, 64);
+    conv<64, false, true>(net, V3, net->p2, Ly[2].wf, P + Ly[2].b_off, nullptr, net->e3, 128);
+    conv<128, true, true>(net, V2, net->e3, Ly[3].wf, P + Ly[3].b_off, net->e2, net->d2, 64);
+    conv<64, true, true>(net, V1, net->d2, Ly[4].wf, P + Ly[4].b_off, net->e1, net->d1, 32);
     hipLaunchKernelGGL(k_head, dim3(gridn(V1.n())), dim3(256), 0, net->stream, V1.n(), net->d1, P + net->h_off,
                        P + net->hb_off, net->y);
 }
@@ -164,38 +180,33 @@ static void backward(pf_net* net, const float* t, const float* wz) {
     Layer* Ly = net->layer;
     float* P = net->p;
     float* G = net->g;
-    hipLaunchKernelGGL(k_loss, dim3(gridn(V1.n(), 256, 2048)), dim3(256), 0, net->stream, V1, net->y, t, net->mask, wz,
+    hipLaunchKernelGGL(k_loss, dim3(gridn(V1.n(), 256, 512)), dim3(256), 0, net->stream, V1, net->y, t, net->mask, wz,
                        net->mask_norm, net->lambda, net->gy, net->dloss);
-    hipLaunchKernelGGL(k_head_bwd, dim3(gridn(V1.n(), 256, 1024)), dim3(256), 0, net->stream, V1.n(), net->gy,
+    hipLaunchKernelGGL(k_head_bwd, dim3(gridn(V1.n() * 4, 256, 256)), dim3(256), 0, net->stream, V1.n(), net->gy,
                        net->d1, P + net->h_off, net->g5, G + net->h_off, G + net->hb_off);
     // C5: d1 = relu(C5(up(d2)) + b5 + e1); g5 = gradient of its pre-activation
-    chan_sum(net, V1.n(), 32, net->g5, G + Ly[4].b_off);
-    wgrad<true>(net, V1, net->g5, net->d2, G + Ly[4].w_off, 32, 64);
-    conv<false, false>(net, V1, 32, net->g5, Ly[4].wt, nullptr, nullptr, net->gu1, 64);
-    hipLaunchKernelGGL(k_up_bwd, dim3(gridn(V2.n() * 64)), dim3(256), 0, net->stream, V2, net->gu1, net->g4, 64,
+    wgrad<64, true>(net, V1, net->g5, net->d2, G + Ly[4].w_off, 32);
+    conv<32, false, false>(net, V1, net->g5, Ly[4].wt, nullptr, nullptr, net->gu1, 64);
+    hipLaunchKernelGGL(k_up_bwd, dim3(gridn(V2.n() * 8)), dim3(256), 0, net->stream, V2, net->gu1, net->g4, 64,
                        net->d2);
     // C4: d2 = relu(C4(up(e3)) + b4 + e2)
-    chan_sum(net, V2.n(), 64, net->g4, G + Ly[3].b_off);
-    wgrad<true>(net, V2, net->g4, net->e3, G + Ly[3].w_off, 64, 128);
-    conv<false, false>(net, V2, 64, net->g4, Ly[3].wt, nullptr, nullptr, net->gu2, 128);
-    hipLaunchKernelGGL(k_up_bwd, dim3(gridn(V3.n() * 128)), dim3(256), 0, net->stream, V3, net->gu2, net->g3, 128,
+    wgrad<128, true>(net, V2, net->g4, net->e3, G + Ly[3].w_off, 64);
+    conv<64, false, false>(net, V2, net->g4, Ly[3].wt, nullptr, nullptr, net->gu2, 128);
+    hipLaunchKernelGGL(k_up_bwd, dim3(gridn(V3.n() * 16)), dim3(256), 0, net->stream, V3, net->gu2, net->g3, 128,
                        net->e3);
     // C3: e3 = relu(C3(p2) + b3)
-    chan_sum(net, V3.n(), 128, net->g3, G + Ly[2].b_off);
-    wgrad<false>(net, V3, net->g3, net->p2, G + Ly[2].w_off, 128, 64);
-    conv<false, false>(net, V3, 128, net->g3, Ly[2].wt, nullptr, nullptr, net->gp2, 64);
+    wgrad<64, false>(net, V3, net->g3, net->p2, G + Ly[2].w_off, 128);
+    conv<128, false, false>(net, V3, net->g3, Ly[2].wt, nullptr, nullptr, net->gp2, 64);
     // e2 feeds the skip of d2 (gradient g4) and pool -> p2 (gradient gp2); in place into g4
-    hipLaunchKernelGGL(k_skip_pool_bwd, dim3(gridn(V2.n() * 64)), dim3(256), 0, net->stream, V2, net->g4, net->gp2,
+    hipLaunchKernelGGL(k_skip_pool_bwd, dim3(gridn(V2.n() * 8)), dim3(256), 0, net->stream, V2, net->g4, net->gp2,
                        net->e2, net->g4, 64);
     // C2: e2 = relu(C2(p1) + b2)
-    chan_sum(net, V2.n(), 64, net->g4, G + Ly[1].b_off);
-    wgrad<false>(net, V2, net->g4, net->p1, G + Ly[1].w_off, 64, 32);
-    conv<false, false>(net, V2, 64, net->g4, Ly[1].wt, nullptr, nullptr, net->gp1, 32);
-    hipLaunchKernelGGL(k_skip_pool_bwd, dim3(gridn(V1.n() * 32)), dim3(256), 0, net->stream, V1, net->g5, net->gp1,
+    wgrad<32, false>(net, V2, net->g4, net->p1, G + Ly[1].w_off, 64);
+    conv<64, false, false>(net, V2, net->g4, Ly[1].wt, nullptr, nullptr, net->gp1, 32);
+    hipLaunchKernelGGL(k_skip_pool_bwd, dim3(gridn(V1.n() * 4)), dim3(256), 0, net->stream, V1, net->g5, net->gp1,
                        net->e1, net->g5, 32);
     // C1: e1 = relu(C1(x) + b1)
-    chan_sum(net, V1.n(), 32, net->g5, G + Ly[0].b_off);
-    wgrad<false>(net, V1, net->g5, net->x, G + Ly[0].w_off, 32, NIN);
+    wgrad<NIN, false>(net, V1, net->g5, net->x, G + Ly[0].w_off, 32);
 }
 
 static int upload_feat(pf_net* net, const float* feat) {
@@ -254,8 +265,8 @@ int pf_net_create(pf_net** out, int device, int nx, int ny, int nz, int max_samp
         if ((rc = nalloc(net, pp, net->nparams))) return bail(rc);
     for (int l = 0; l < 5; ++l) {
         Layer& L = net->layer[l];
-        if ((rc = nalloc(net, &L.wf, 27 * (size_t)L.cin * L.cout))) return bail(rc);
-        if (l > 0 && (rc = nalloc(net, &L.wt, 27 * (size_t)L.cin * L.cout))) return bail(rc);
+        if ((rc = nalloc(net, &L.wf, frag_size(L.cin, L.cout)))) return bail(rc);
+        if (l > 0 && (rc = nalloc(net, &L.wt, frag_size(L.cout, L.cin)))) return bail(rc);
     }
     const size_t n1 = net->L[0].n(), n2 = net->L[1].n(), n3 = net->L[2].n();
     struct {
@@ -274,6 +285,10 @@ int pf_net_create(pf_net** out, int device, int nx, int ny, int nz, int max_samp
     if ((rc = nalloc(net, &net->dloss, 1))) return bail(rc);
     net->max_samples = max_samples;
     if (max_samples) {
+        const Vol &V1 = net->L[0], &V2 = net->L[1], &V3 = net->L[2];
+        const size_t np = std::max({wgrad_part<64, true>(V1, 32), wgrad_part<128, true>(V2, 64), wgrad_part<64, false>(V3, 128),
+                                    wgrad_part<32, false>(V2, 64), wgrad_part<NIN, false>(V1, 32)});
+        if ((rc = nalloc(net, &net->part, np))) return bail(rc);
         if ((rc = nalloc(net, &net->dfeat, n1 * NIN * (size_t)max_samples))) return bail(rc);
         if ((rc = nalloc(net, &net->dtarget, n1 * (size_t)max_samples))) return bail(rc);
     }
