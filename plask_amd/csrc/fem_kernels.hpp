@@ -1478,6 +1478,32 @@ __host__ __device__ inline int part_lds_values(int P, int CB, int S) {
     return 6 * (S + (part_scan_width(P, CB, S) ? P : 0));
 }
 
+// The line factors of a thread's segment: a and w of every plane; c' only of the separator
+// (its coupling upwards), the interior ones are c'_u = a_(u+1) w_u (the coupling to the next
+// interior plane times the pivot inverse, as the set-up forms them), 0 on the last.
+template <typename T, int M>
+__device__ __forceinline__ void part_factors(const PartPos& q, long long plane, const T* __restrict__ la,
+                                             const T* __restrict__ lw, const T* __restrict__ lcp, T (&av)[M], T (&wv)[M],
+                                             T (&cv)[M]) {
+    T cs = T(0);
+    if (q.sep) cs = lcp[q.base + (long long)(q.len - 1) * plane];
+#pragma unroll
+    for (int u = 0; u < M; ++u) {
+        av[u] = wv[u] = T(0);
+        if (u < q.len) {
+            const long long node = q.base + (long long)u * plane;
+            av[u] = la[node];
+            wv[u] = lw[node];
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < M; ++u) {
+        cv[u] = T(0);
+        if (u + 1 < M) cv[u] = u + 1 < q.lint ? av[u + 1] * wv[u] : T(0);
+        if (q.sep && u == q.len - 1) cv[u] = cs;
+    }
+}
+
 // z = T^-1 r for the thread's segment (values in registers): interior solve
 // y = T_j^-1 r; the separator right-hand sides g = r_s - T_sI y go to LDS; S z_s = g is
 // solved per column (a shuffle scan, or one thread); each interior is solved again with the separator
@@ -1498,10 +1524,10 @@ __device__ inline void part_solve(const PartPos& q, int P, int CB, int ncol, con
     T* s_sc = s_sw + SP;
     const int t = q.t, cl = q.cl, seg = q.seg;
     const int pt = seg * CS + cl;  // the thread's slot (threads past CB * P have none)
-    if (q.sep) {
-        s_sa[pt] = schur[(size_t)seg * ncol + q.col];
-        s_sw[pt] = schur[(size_t)(P - 1 + seg) * ncol + q.col];
-        s_sc[pt] = schur[(size_t)(2 * (P - 1) + seg) * ncol + q.col];
+    if (seg < P - 1) {  // zero for the columns past the grid
+        s_sa[pt] = q.sep ? schur[(size_t)seg * ncol + q.col] : T(0);
+        s_sw[pt] = q.sep ? schur[(size_t)(P - 1 + seg) * ncol + q.col] : T(0);
+        s_sc[pt] = q.sep ? schur[(size_t)(2 * (P - 1) + seg) * ncol + q.col] : T(0);
     }
     // interior solve with the separators at zero
     T d[M];
@@ -1548,7 +1574,7 @@ __device__ inline void part_solve(const PartPos& q, int P, int CB, int ncol, con
     const int ns = P - 1;
     if (W) {
         const int j = t & (W - 1), c = t / W;
-        const bool on = j < ns && c < CB && q.col - cl + c < ncol;
+        const bool on = j < ns && c < CB;
         const int o = j * CS + c;
         T a = T(0), b = T(0);
         if (on) {
@@ -1573,7 +1599,7 @@ __device__ inline void part_solve(const PartPos& q, int P, int CB, int ncol, con
             }
         }
         if (on) s_g[o] = b;
-    } else if (seg == 0 && q.col < ncol) {
+    } else if (seg == 0 && q.act) {
         T dq = T(0);
         for (int j = 0; j < P - 1; ++j) {
             const int o = j * CS + cl;
@@ -1636,12 +1662,10 @@ __global__ __launch_bounds__((PartLB<T, M>::value)) void k_cg_part(
         if (u < pp.len) {
             const long long node = pp.base + (long long)u * plane;
             rv[u] = r[node];
-            av[u] = la[node];
-            wv[u] = lw[node];
-            cv[u] = lcp[node];
             if (!START) qv[u] = q[node];
         }
     }
+    part_factors<T, M>(pp, plane, la, lw, lcp, av, wv, cv);
     const T alpha = START ? T(0) : T(st->alpha);
     double rr = 0., rz = 0.;
 #pragma unroll
@@ -1755,15 +1779,13 @@ __global__ __launch_bounds__((PartLB<T, M>::value)) void k_mg_smooth(
             } else {
                 rv[u] = r[node];
             }
-            av[u] = la[node];
-            wv[u] = lw[node];
-            cv[u] = lcp[node];
             if (UPD) {
                 rv[u] = rv[u] - alpha * q[node];
                 r[node] = rv[u];
             }
         }
     }
+    part_factors<T, M>(pp, plane, la, lw, lcp, av, wv, cv);
     T zv[M];
     part_solve<T, M>(pp, P, CB, ncol, schur, reinterpret_cast<T*>(part_smem), rv, av, wv, cv, zv);
     double rz = 0., rr = 0.;

@@ -292,13 +292,13 @@ static double mask_bytes(long long n) { return 8.0 * (double)((n + 63) / 64); }
 static double bytes_apply_fused(long long n, long long e, int t) { return t * (6.0 * n + 2.0 * e) + mask_bytes(n); }
 // residual r = b - A x: x, b read; r written
 static double bytes_residual(long long n, long long e, int t) { return t * (3.0 * n + 2.0 * e) + mask_bytes(n); }
-// damped line sweep: right-hand side and the three line factors read, the sweep written;
+// damped line sweep: right-hand side and two line factors read, the sweep written;
 // with the PCG update also q read and the right-hand side written back; a previous
 // iterate read when there is one; the PCG residual read for the final dot products;
-// three factors per separator and column
+// four factors per separator and column
 static double bytes_smooth(long long n, int ncol, int P, int t, bool upd, bool xin, bool fin) {
-    const double v = 5.0 + (upd ? 2.0 : 0.0) + (xin ? 1.0 : 0.0) + (fin && !upd ? 1.0 : 0.0);
-    return t * (v * n + 3.0 * std::max(P - 1, 0) * (double)ncol);
+    const double v = 4.0 + (upd ? 2.0 : 0.0) + (xin ? 1.0 : 0.0) + (fin && !upd ? 1.0 : 0.0);
+    return t * (v * n + 4.0 * std::max(P - 1, 0) * (double)ncol);
 }
 
 static void prof_close(pf_ctx* ctx, int h) {
@@ -386,6 +386,12 @@ static int part_lb(int m) {
     return 0;
 }
 
+static int part_threads(int P, int lb) {
+    int W = 1;
+    while (W < P - 1) W <<= 1;
+    return W <= 64 && W <= lb ? std::max(P, W) : P;
+}
+
 template <typename T>
 static PartShape part_shape(int m, int n, int ncol) {
     PartShape ps;
@@ -397,10 +403,14 @@ static PartShape part_shape(int m, int n, int ncol) {
         ps.m = 0;
         return ps;
     }
+    // threads per column: its segments, or the lanes of its separator scan where that is more
+    // (a power of two, at most 64); without room for the scan's lanes one thread would walk
+    // the separators (24 segments at 192 planes: 23 dependent LDS steps each way)
+    const int per = part_threads(ps.P, lb);
     ps.CB = 64;
-    while (ps.CB > 1 && ps.CB * ps.P > lb) ps.CB >>= 1;
+    while (ps.CB > 1 && ps.CB * per > lb) ps.CB >>= 1;
     while (ps.CB > 1 && ps.CB / 2 >= ncol) ps.CB >>= 1;
-    ps.threads = (ps.CB * ps.P + 63) / 64 * 64;
+    ps.threads = (ps.CB * per + 63) / 64 * 64;
     return ps;
 }
 
@@ -544,6 +554,40 @@ static size_t tile_lds(int rows, int n0) {
     return sizeof(double) * (size_t)(2 * (rows + 1) + 8 * rows) * (size_t)(n0 + 1);
 }
 
+// Rows per block of the 3D tile kernel: as many as 512 threads and 64 KiB of LDS hold (at
+// most 16), or fewer where that saves waves per z-chunk (tiles x waves per tile; ties keep
+// the larger tile): 17 x 17 columns take 11 rows (2 tiles of 3 waves), not 16 (2 of 5).
+static int tile_rows(int n0, int n1) {
+    int BY = std::max(2, std::min(16, 512 / n0));
+    while (BY > 2 && (BY * n0 > 1024 || tile_lds(BY, n0) > 65536)) --BY;
+    int best = BY;
+    long long cost = -1;
+    for (int by = std::min(BY, n1 + 1); by >= 2; --by) {
+        const long long c = (long long)((n1 + by - 2) / (by - 1)) * ((by * n0 + 63) / 64);
+        if (cost < 0 || c < cost) {
+            cost = c;
+            best = by;
+        }
+    }
+    return best;
+}
+
+// Planes per block: kmax, halved until the grid has about 2 blocks per CU (aiming at 4 measured
+// slower: 65 x 65 columns 22.0 against 17.7 us per launch).
+static int tile_planes(int BY, int n1, int n2, int kmax) {
+    const long long ytiles = (n1 + BY - 2) / (BY - 1);
+    int KC = kmax;
+    while (KC > 1 && (KC > n2 || ytiles * ((n2 + KC - 1) / KC) < 512)) KC >>= 1;
+    return KC;
+}
+
+// 2D: rows of axis 1 per block, short enough for about one block per CU
+static int rows2d(int n1) {
+    int KC = 64;
+    while (KC > 1 && (n1 + KC - 1) / KC < 256) KC >>= 1;
+    return KC;
+}
+
 int pf_grid_set(pf_ctx* ctx, int dim, int geom, const double* ax0, int64_t n0, const double* ax1, int64_t n1,
                 const double* ax2, int64_t n2) {
     if (!ctx) return PF_EINVAL;
@@ -653,20 +697,22 @@ int pf_grid_set(pf_ctx* ctx, int dim, int geom, const double* ax0, int64_t n0, c
     ctx->have_coeffs = false;
     ctx->have_source = false;
     ctx->have_solution = false;
-    // launch shapes: tile blocks of BY node rows (BY - 1 owned) x whole x rows, KC planes;
-    // measured best at 128 x 128 x 256: 4 rows, 16 planes in both precisions (FP64: 8.23 ms
-    // per multigrid solve against 8.32 with 8 planes, 8.47 with 32, 8.32 with 6 rows; a
-    // prefetch depth of 2 planes is slower, 8.52)
+    // launch shapes: tile blocks of BY node rows (BY - 1 owned) x whole x rows, KC planes.  On
+    // large grids 4 rows x 16 planes (measured best at 128 x 128 x 256: FP64 8.23 ms per
+    // multigrid solve against 8.32 with 8 planes, 8.47 with 32, 8.32 with 6 rows; a prefetch
+    // depth of 2 planes is slower, 8.52).  Small grids are held by the latency of the z-march
+    // (about 1 us per plane): shorter marches until there are about two blocks per CU, as on
+    // the multigrid's coarse levels (25 x 19 x 37 nodes: the fused apply 19.5 us with 16 planes
+    // per block, 6 with 1; 48 x 48 x 96: 23.7 and 8).
     if (dim == 3) {
-        const int by = (int)std::max<int64_t>(2, std::min<int64_t>(16, 512 / n0));
+        const int by = tile_rows((int)n0, (int)n1);
         ctx->BY[0] = ctx->BY[1] = by;
-        ctx->KC[0] = (int)std::max<int64_t>(1, std::min<int64_t>(16, n2));
-        ctx->KC[1] = (int)std::max<int64_t>(1, std::min<int64_t>(16, n2));
+        ctx->KC[0] = ctx->KC[1] = tile_planes(by, (int)n1, (int)n2, 16);
         // long x rows: the tile kernel's LDS would pass 64 KiB, use row blocks
         const int kind = tile_lds(by, (int)n0) > 65536 ? 1 : 0;
         ctx->apply_kind[0] = ctx->apply_kind[1] = kind;
     } else {
-        ctx->KC2 = (int)std::max<int64_t>(4, std::min<int64_t>(64, n1 / 64));
+        ctx->KC2 = rows2d((int)n1);
     }
     ctx->upd_blocks = grid1(N, 256, 1024);
     size_t napply = 0;
@@ -1526,8 +1572,7 @@ static void mg_residual_launch(pf_ctx* ctx, int l, const MgView<T>& v, MgProl<T>
         // one block per chunk of KC rows of the layer axis, one thread per node of axis 0;
         // short chunks on the (latency-bound) coarse levels
         const int n0 = v.g2.n0, n1 = v.g2.n1;
-        int KC = 64;
-        while (KC > 1 && (n1 + KC - 1) / KC < 256) KC >>= 1;
+        const int KC = rows2d(n1);
         pf_launch(ctx, (k_apply2d<T, MODE_RESG, false, false>), dim3((n1 + KC - 1) / KC), dim3(n0),
                            sizeof(T) * 4 * (size_t)(n0 + 1), ctx->stream, v.g2, KC, (const T*)v.x, (const T*)nullptr,
                            (const T*)nullptr, (T*)nullptr, (T*)nullptr, v.r, (const T*)v.b, v.dmask, v.kh, v.kv,
@@ -1535,27 +1580,9 @@ static void mg_residual_launch(pf_ctx* ctx, int l, const MgView<T>& v, MgProl<T>
         return;
     }
     const int n0 = v.g.n0, n1 = v.g.n1, n2 = v.g.n2;
-    int BY = std::max(2, std::min(16, 512 / n0));
-    while (BY > 2 && (BY * n0 > 1024 || tile_lds(BY, n0) > 65536)) --BY;
-    {  // fewer rows where that saves waves per z-chunk (tiles x waves per tile; ties keep
-       // the larger tile): 17 x 17 columns take 11 rows (2 tiles of 3 waves), not 16 (2 of 5)
-        int best = BY;
-        long long cost = -1;
-        for (int by = std::min(BY, n1 + 1); by >= 2; --by) {
-            const long long c = (long long)((n1 + by - 2) / (by - 1)) * ((by * n0 + 63) / 64);
-            if (cost < 0 || c < cost) {
-                cost = c;
-                best = by;
-            }
-        }
-        BY = best;
-    }
+    const int BY = tile_rows(n0, n1);
     const int ytiles = (n1 + BY - 2) / (BY - 1);
-    // coarse levels are latency-bound: shorter z-marches (down to 1 plane per block)
-    // until the grid has about 2 blocks per CU (aiming at 4 measured slower: 65 x 65
-    // columns 22.0 against 17.7 us per launch)
-    int KC = 8;
-    while (KC > 1 && (long long)ytiles * ((n2 + KC - 1) / KC) < 512) KC >>= 1;
+    const int KC = tile_planes(BY, n1, n2, 8);
     const int nb = ytiles * ((n2 + KC - 1) / KC), grid = (nb + 7) / 8 * 8;
     const size_t shm = tile_lds(BY, n0) / sizeof(double) * sizeof(T);
     const int xo = ctx->mg_xcd ? 2 : ctx->xcd_order;
@@ -1615,7 +1642,7 @@ static void mg_smooth(pf_ctx* ctx, const MgView<T>& v, bool upd, int fin, T* r, 
     // at least 64 blocks (larger levels keep full blocks, which measured faster)
     while (ps.CB > 4 && (ncol + ps.CB - 1) / ps.CB < 64) {
         ps.CB >>= 1;
-        ps.threads = (ps.CB * ps.P + 63) / 64 * 64;
+        ps.threads = (ps.CB * part_threads(ps.P, 1024) + 63) / 64 * 64;
     }
     // coarse levels with the XCD-aligned order: the grid a multiple of 8 (idle blocks
     // past the last column group)
@@ -1829,7 +1856,7 @@ static int run_cg(pf_ctx* ctx, int precond, T* x, T* r, T* p, T* p2, T* q, T* z,
         } else if (mg) {
             mg_vcycle<T>(ctx, r, q, z, true, 1);
         } else if (line && pm) {
-            hk = prof_kern<T>(ctx, PF_K_LINE, 0, tb * (7.0 * N + 3.0 * std::max(ps.P - 1, 0) * (double)ncol));
+            hk = prof_kern<T>(ctx, PF_K_LINE, 0, tb * (6.0 * N + 4.0 * std::max(ps.P - 1, 0) * (double)ncol));
             launch_part<T, false>(ctx, ps, ncol, nplanes, plane, r, q, la, lw, lcp, schur, z);
         } else if (line) {
             hk = prof_kern<T>(ctx, PF_K_LINE, 0, tb * 9.0 * N);
