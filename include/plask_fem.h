@@ -261,7 +261,8 @@ int pf_set_launch(pf_ctx* ctx, int rows, int planes);
  * the Schur complement of the segment separators (FP64 uses at most 16), on every
  * multigrid level; seg = 0 restores the default (8 FP64, 16 FP32 on the solve grid;
  * the multigrid coarse levels take 8, and 4 on levels of at most 512 columns, where
- * the separators stay at most 64); seg < 0 selects the sequential one-thread-per-line
+ * the separators stay at most 64).  Up to 128 separators of a line are solved by a shuffle
+ * scan, more by one thread per line; seg < 0 selects the sequential one-thread-per-line
  * kernel.  No counterpart in the reference (a tuning hook). */
 int pf_set_line_segment(pf_ctx* ctx, int seg);
 
@@ -487,11 +488,14 @@ int pf_get_currents(pf_ctx* ctx, double* cur, double* heat);
 
 /* Batched uneven 2D Shockley problems --------------------------------------
  * Many independent ElectricalFem2DSolver::compute runs (electr2d.cpp:363-440, junction
- * law beta.hpp:43-46) -- e.g. voltage/temperature sweeps over device variants -- in one
- * persistent kernel launch replayed from a hipGraph.  Each workgroup takes instances
- * from a largest-first work queue and runs the whole Picard loop on the device: junction
- * update, line- or multigrid-preconditioned CG (warm start), currents and loop error.  The reference
- * runs such sweeps as separate processes (gui/plugins/launcher_batch.py:16). */
+ * law beta.hpp:43-46) -- e.g. voltage/temperature sweeps over device variants.  With the
+ * multigrid preconditioner all instances advance together, one launch per step over the blocks of
+ * those that have not ended, replayed from hipGraphs.  With the line preconditioner, and where a
+ * mesh has more than 1032 rows of axis 1 or more than 2049 columns, one persistent kernel: each
+ * workgroup takes instances from a largest-first work queue and runs the whole Picard loop.  Either
+ * way the loop runs on the device: junction update, preconditioned CG (warm start), currents and
+ * loop error.  The reference runs such sweeps as separate processes
+ * (gui/plugins/launcher_batch.py:16). */
 typedef struct pf_batch pf_batch;
 
 typedef struct {
@@ -506,15 +510,15 @@ typedef struct {
                        with conductivities spanning ~1e14 -- has the potential FP64 CG reaches; `rel` and `bwd`
                        report it) */
     int stable;     /* CONVERGENCE_STABLE */
-    int block;      /* threads per workgroup 256/512/1024; 0 = autotuned or 1024 */
-    int nwg;        /* persistent workgroups; 0 = autotuned or one per CU */
+    int block;      /* persistent kernel: threads per workgroup 256/512/1024; 0 = autotuned or 1024 */
+    int nwg;        /* persistent kernel: workgroups; 0 = autotuned or one per CU */
     int precond;    /* 3 (or 0, the default) = multigrid V-cycle (axis 0 coarsened per instance,
                        damped line smoother, omega 0.65, 2 coarsest sweeps); 2 = line preconditioner */
-    int loop_budget;/* Picard loops one kernel launch runs per instance (0: all of them in one launch).
-                       The solve relaunches the kernel until every instance has finished, so a
-                       launch returns after a bounded amount of work whatever the batch */
-    /* called between launches (may be NULL): launches so far, instances finished, total,
-       seconds since the first launch, progress_user */
+    int loop_budget;/* Picard loops between two calls of progress (0: one call, at the end).  The
+                       persistent kernel is relaunched after that many loops per instance, so that
+                       a launch returns after a bounded amount of work whatever the batch */
+    /* called after every loop_budget loops (may be NULL): calls so far, instances finished,
+       total, seconds since the first launch, progress_user */
     void (*progress)(int launches, int finished, int total, double seconds, void* user);
     void* progress_user;
 } pf_batch_opts;
@@ -540,11 +544,12 @@ const char* pf_batch_last_error(const pf_batch* b);
 int pf_batch_set(pf_batch* b, int ninst, int cylindrical, const int32_t* n0, const int32_t* n1, const double* ax0,
                  const double* ax1, const double* sh, const double* sv, const int64_t* ndir, const int64_t* dnodes,
                  const double* dvals, const int32_t* jlo, const int32_t* jhi, const double* beta, const double* js);
-/* Times each (block, workgroups) schedule on the batch and keeps the fastest. */
+/* Times each (block, workgroups) schedule of the persistent kernel on the batch and keeps the
+ * fastest; where all instances advance together there is no such choice and one run is timed. */
 int pf_batch_autotune(pf_batch* b, const pf_batch_opts* o, int* best_block, int* best_nwg, double* best_seconds);
 /* Solve every instance from V = Dirichlet values / 0; V_out (concatenated, may be NULL),
- * stats[ninst] (may be NULL), seconds = device time of all launches (the start launch and
- * every launch of the persistent kernel, with the host's progress reads between them).
+ * stats[ninst] (may be NULL), seconds = device time of all launches, with the host's
+ * progress reads between them.
  * The launches are replayed from hipGraphs (plain launches under a kernel-tracing
  * profiler, as for pf_solve). */
 int pf_batch_solve(pf_batch* b, const pf_batch_opts* o, double* V_out, pf_batch_stats* stats, double* seconds);

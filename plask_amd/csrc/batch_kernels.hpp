@@ -139,25 +139,20 @@ __device__ __forceinline__ bool lbit(const LView& V, long long node) { return db
 // are issued before the current row is formed.  Element matrix of therm2d.cpp:225-228 /
 // electr2d.cpp:296-304 (x r_mid for cylindrical geometry), summed element by element.
 // KIND 0: y = M A0 M x + (I - M) x; returns the sum of x y over the rows formed;
-// KIND 1: y = b + M (0 - A0 x) (b null: 0); returns 0;
+// KIND 1: y = b + M (0 - A0 x) (b null: 0); returns the sum of y^2;
 // KIND 2: y = M (0 - A0 x) with the products and their sum carried in double-double (Dot2):
 //   the residual of a nearly converged potential is then accurate to about the rounding of
 //   the result, not to eps |A0| |x|, so CG restarted from it can reduce the true residual
 //   below the level its recursive residual drifts to; returns the sum of y^2, and bw the max
 //   over the rows of |y_i| / (|A0| |x|)_i (no FP64 potential has a residual much below eps
 //   times that row).
-template <int BS, int KIND>
-__device__ inline double march_l(const LView& V, const double* __restrict__ x, const double* __restrict__ b,
-                                 double* __restrict__ y, double& bw) {
+template <int KIND>
+__device__ __forceinline__ double march_rows(const LView& V, int i, int k0, int k1, const double* __restrict__ x,
+                                             const double* __restrict__ b, double* __restrict__ y, double& bw) {
     const int n0 = V.n0, n1 = V.n1;
-    const int G = n0 >= BS ? 1 : BS / n0;  // row ranges per column
-    const int R = (n1 + G - 1) / G;
     double acc = 0.;
     bw = 0.;
-    for (int w = threadIdx.x; w < G * n0; w += BS) {
-        const int g = w / n0, i = w - g * n0;
-        const int k0 = g * R, k1 = min(n1, k0 + R);
-        if (k0 >= k1) continue;
+    {
         const bool eL = i >= 1, eR = i < n0 - 1;
         const int im = max(i - 1, 0), ip = min(i + 1, n0 - 1);
         const int eiL = max(i - 1, 0), eiR = min(i, n0 - 2);
@@ -259,6 +254,7 @@ __device__ inline double march_l(const LView& V, const double* __restrict__ x, c
                     acc += xw[1][1] * out;
                 } else {
                     out = (b ? b[node] : 0.) + (di ? 0. : -s);
+                    acc += out * out;
                 }
             }
             y[node] = out;
@@ -274,6 +270,25 @@ __device__ inline double march_l(const LView& V, const double* __restrict__ x, c
             for (int d = 0; d < 4; ++d) ke[0][d] = ke[1][d];
             he[0] = he[1];
         }
+    }
+    return acc;
+}
+
+template <int BS, int KIND>
+__device__ inline double march_l(const LView& V, const double* __restrict__ x, const double* __restrict__ b,
+                                 double* __restrict__ y, double& bw) {
+    const int n0 = V.n0, n1 = V.n1;
+    const int G = n0 >= BS ? 1 : BS / n0;  // row ranges per column
+    const int R = (n1 + G - 1) / G;
+    double acc = 0.;
+    bw = 0.;
+    for (int w = threadIdx.x; w < G * n0; w += BS) {
+        const int g = w / n0, i = w - g * n0;
+        const int k0 = g * R, k1 = min(n1, k0 + R);
+        if (k0 >= k1) continue;
+        double bwi;
+        acc += march_rows<KIND>(V, i, k0, k1, x, b, y, bwi);
+        bw = fmax(bw, bwi);
     }
     return acc;
 }

@@ -1220,7 +1220,7 @@ __global__ void k_line_setup2d(Axes2<double> g, const double* __restrict__ kh, c
 // T_II is block diagonal (one tridiagonal block per interior), so each segment
 // is solved by its own thread with its planes held in registers; the small S system
 // of each column is then solved from its Thomas factors (by a shuffle scan over the
-// separators, or one thread's walk for lines of more than 64 separators; part_solve).
+// separators, or one thread's walk for lines of more than 128 separators; part_solve).
 // Stored per node:
 //   interior plane: la = coupling to the previous interior plane (0 on the
 //     first), lw = LDL^T pivot inverse, lcp = c' (0 on the last);
@@ -1267,7 +1267,52 @@ __global__ void k_line_bc2d(Axes2<double> g, const double* __restrict__ kh, cons
     }
 }
 
-// thread = (column, segment); sff / sfl: [segment][column] (segment 0 unused)
+// interior factors of segment s of a column and (s > 0) its sums, sff / sfl: [segment][column]
+template <typename T>
+__device__ inline void part_factor_segment(int col, int s, int ncol, int n, int m, long long plane,
+                                           const double* __restrict__ bb, const double* __restrict__ cc,
+                                           T* __restrict__ la, T* __restrict__ lw, T* __restrict__ lcp,
+                                           double* __restrict__ sff, double* __restrict__ sfl) {
+    const int P = (n + m - 1) / m;
+    const int k0 = s * m, k1 = min(k0 + m, n);
+    double cprev = 0., cpprev = 0.;
+    for (int k = k0; k < k1; ++k) {
+        const long long node = (long long)k * plane + col;
+        const double b = bb[node], c = cc[node];
+        const int u = k - k0;
+        if (u == m - 1 && s < P - 1) {  // separator
+            la[node] = T(cprev);
+            lw[node] = T(b);
+            lcp[node] = T(c);
+        } else {
+            const bool last = s < P - 1 ? u == m - 2 : k == n - 1;
+            const double a = u == 0 ? 0. : cprev;
+            const double w = 1. / (b - a * cpprev);
+            const double cp = last ? 0. : c * w;
+            la[node] = T(a);
+            lw[node] = T(w);
+            lcp[node] = T(cp);
+            cprev = c;
+            cpprev = cp;
+        }
+    }
+    if (s == 0) return;
+    // interior of this segment (what follows the separator of segment s - 1), from
+    // the stored (precision T) factors as the separator step reads them
+    const int ke = s < P - 1 ? k0 + m - 1 : n;
+    double v = 1., ff = 0., wprev = 0.;
+    for (int k = k0; k < ke; ++k) {
+        const long long node = (long long)k * plane + col;
+        const double w = lw[node];
+        if (k > k0) v = -(double)la[node] * wprev * v;
+        ff += v * v * w;
+        wprev = w;
+    }
+    sff[(size_t)s * ncol + col] = ff;
+    sfl[(size_t)s * ncol + col] = v * wprev;
+}
+
+// thread = (column, segment)
 template <typename T>
 __global__ void k_part_factor(int ncol, int n, int m, long long plane, const double* __restrict__ bb,
                               const double* __restrict__ cc, T* __restrict__ la, T* __restrict__ lw,
@@ -1275,53 +1320,16 @@ __global__ void k_part_factor(int ncol, int n, int m, long long plane, const dou
     const int P = (n + m - 1) / m;
     const long long total = (long long)P * ncol;
     for (long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x; t < total;
-         t += (long long)gridDim.x * blockDim.x) {
-        const int col = (int)(t % ncol), s = (int)(t / ncol);
-        const int k0 = s * m, k1 = min(k0 + m, n);
-        double cprev = 0., cpprev = 0.;
-        for (int k = k0; k < k1; ++k) {
-            const long long node = (long long)k * plane + col;
-            const double b = bb[node], c = cc[node];
-            const int u = k - k0;
-            if (u == m - 1 && s < P - 1) {  // separator
-                la[node] = T(cprev);
-                lw[node] = T(b);
-                lcp[node] = T(c);
-            } else {
-                const bool last = s < P - 1 ? u == m - 2 : k == n - 1;
-                const double a = u == 0 ? 0. : cprev;
-                const double w = 1. / (b - a * cpprev);
-                const double cp = last ? 0. : c * w;
-                la[node] = T(a);
-                lw[node] = T(w);
-                lcp[node] = T(cp);
-                cprev = c;
-                cpprev = cp;
-            }
-        }
-        if (s == 0) continue;
-        // interior of this segment (what follows the separator of segment s - 1), from
-        // the stored (precision T) factors as the separator step reads them
-        const int ke = s < P - 1 ? k0 + m - 1 : n;
-        double v = 1., ff = 0., wprev = 0.;
-        for (int k = k0; k < ke; ++k) {
-            const long long node = (long long)k * plane + col;
-            const double w = lw[node];
-            if (k > k0) v = -(double)la[node] * wprev * v;
-            ff += v * v * w;
-            wprev = w;
-        }
-        sff[(size_t)s * ncol + col] = ff;
-        sfl[(size_t)s * ncol + col] = v * wprev;
-    }
+         t += (long long)gridDim.x * blockDim.x)
+        part_factor_segment<T>((int)(t % ncol), (int)(t / ncol), ncol, n, m, plane, bb, cc, la, lw, lcp, sff, sfl);
 }
 
+// LU recurrence of a column's separator system
 template <typename T>
-__global__ void k_part_schur(int ncol, int n, int m, long long plane, const T* __restrict__ la,
-                             const T* __restrict__ lw, const T* __restrict__ lcp, const double* __restrict__ sff,
-                             const double* __restrict__ sfl, T* __restrict__ schur) {
-    const int col = blockIdx.x * blockDim.x + threadIdx.x;
-    if (col >= ncol) return;
+__device__ inline void part_schur_column(int col, int ncol, int n, int m, long long plane, const T* __restrict__ la,
+                                         const T* __restrict__ lw, const T* __restrict__ lcp,
+                                         const double* __restrict__ sff, const double* __restrict__ sfl,
+                                         T* __restrict__ schur) {
     const int P = (n + m - 1) / m;
     double off_prev = 0., sc_prev = 0.;
     for (int j = 0; j < P - 1; ++j) {
@@ -1339,6 +1347,15 @@ __global__ void k_part_schur(int ncol, int n, int m, long long plane, const T* _
         off_prev = soff;
         sc_prev = cp;
     }
+}
+
+template <typename T>
+__global__ void k_part_schur(int ncol, int n, int m, long long plane, const T* __restrict__ la,
+                             const T* __restrict__ lw, const T* __restrict__ lcp, const double* __restrict__ sff,
+                             const double* __restrict__ sfl, T* __restrict__ schur) {
+    const int col = blockIdx.x * blockDim.x + threadIdx.x;
+    if (col >= ncol) return;
+    part_schur_column<T>(col, ncol, n, m, plane, la, lw, lcp, sff, sfl, schur);
 }
 
 // Column kernel: one thread per line segment (blockIdx.y selects the segment; with
@@ -1464,13 +1481,18 @@ __device__ inline PartPos part_pos(int ncol, int n, int P, int CB, long long pla
     return q;
 }
 
-// Width of the shuffle scan that solves a column's separator system in part_solve (the
-// power of two >= P - 1), or 0 where one thread walks each column instead: more than 64
-// separators, or fewer threads in the block than CB * W.
-__host__ __device__ inline int part_scan_width(int P, int CB, int S) {
+// Width of the shuffle scan that solves a column's separator system in part_solve: the power
+// of two >= P - 1 (up to 64 separators, one per lane) or 64 (up to 128, two per lane), or 0
+// where one thread walks each column instead: more separators, or fewer threads in the block
+// than CB * W.
+__host__ __device__ inline int part_scan_lanes(int P) {
     int W = 1;
-    while (W < P - 1) W <<= 1;
-    return (W <= 64 && CB * W <= S) ? W : 0;
+    while (W < P - 1 && W < 64) W <<= 1;
+    return P - 1 <= 2 * W ? W : 0;
+}
+__host__ __device__ inline int part_scan_width(int P, int CB, int S) {
+    const int W = part_scan_lanes(P);
+    return CB * W <= S ? W : 0;
 }
 
 // LDS values of part_solve for blocks of S threads
@@ -1524,10 +1546,12 @@ __device__ inline void part_solve(const PartPos& q, int P, int CB, int ncol, con
     T* s_sc = s_sw + SP;
     const int t = q.t, cl = q.cl, seg = q.seg;
     const int pt = seg * CS + cl;  // the thread's slot (threads past CB * P have none)
-    if (seg < P - 1) {  // zero for the columns past the grid
-        s_sa[pt] = q.sep ? schur[(size_t)seg * ncol + q.col] : T(0);
-        s_sw[pt] = q.sep ? schur[(size_t)(P - 1 + seg) * ncol + q.col] : T(0);
-        s_sc[pt] = q.sep ? schur[(size_t)(2 * (P - 1) + seg) * ncol + q.col] : T(0);
+    // the separator factors (zero for the columns past the grid) travel while the interior is solved
+    T fa = T(0), fw = T(0), fc = T(0);
+    if (q.sep) {
+        fa = schur[(size_t)seg * ncol + q.col];
+        fw = schur[(size_t)(P - 1 + seg) * ncol + q.col];
+        fc = schur[(size_t)(2 * (P - 1) + seg) * ncol + q.col];
     }
     // interior solve with the separators at zero
     T d[M];
@@ -1558,6 +1582,11 @@ __device__ inline void part_solve(const PartPos& q, int P, int CB, int ncol, con
             elo = av[u];
             ehi = cv[u];
         }
+    if (seg < P - 1) {
+        s_sa[pt] = fa;
+        s_sw[pt] = fw;
+        s_sc[pt] = fc;
+    }
     if (seg < P) {
         s_yf[pt] = q.act ? d[0] : T(0);
         s_g[pt] = q.sep ? rs - elo * yl : T(0);
@@ -1570,18 +1599,27 @@ __device__ inline void part_solve(const PartPos& q, int P, int CB, int ncol, con
     // take one separator each and run both bidiagonal solves as affine first-order
     // recurrences x_j = a_j x_(j-1) + b_j, with a log2(W)-step scan over shuffles
     // ((a, b) after (a', b') composes to (a a', a b' + b)) instead of a walk of P - 1
-    // dependent steps.  Longer lines walk each column with one thread.
+    // dependent steps.  Up to 128: a lane takes two neighbouring separators and scans their
+    // composition.  Still longer lines walk each column with one thread.
     const int ns = P - 1;
     if (W) {
         const int j = t & (W - 1), c = t / W;
-        const bool on = j < ns && c < CB;
-        const int o = j * CS + c;
-        T a = T(0), b = T(0);
+        const bool two = ns > W;  // uniform
+        const int j0 = two ? 2 * j : j;
+        const bool on = j0 < ns && c < CB, on1 = two && j0 + 1 < ns && c < CB;
+        const int o = j0 * CS + c, o1 = o + CS;
+        T a0 = T(0), b0 = T(0), a1 = T(0), b1 = T(0);
         if (on) {
             const T w = s_sw[o];
-            a = -s_sa[o] * w;
-            b = (s_g[o] - s_eh[o] * s_yf[o + CS]) * w;
+            a0 = -s_sa[o] * w;
+            b0 = (s_g[o] - s_eh[o] * s_yf[o + CS]) * w;
         }
+        if (on1) {
+            const T w = s_sw[o1];
+            a1 = -s_sa[o1] * w;
+            b1 = (s_g[o1] - s_eh[o1] * s_yf[o1 + CS]) * w;
+        }
+        T a = two ? a1 * a0 : a0, b = two ? fma(a1, b0, b1) : b0;
         for (int d = 1; d < W; d <<= 1) {  // L y = g
             const T ap = __shfl_up(a, d, W), bp = __shfl_up(b, d, W);
             if (j >= d) {
@@ -1589,14 +1627,29 @@ __device__ inline void part_solve(const PartPos& q, int P, int CB, int ncol, con
                 a *= ap;
             }
         }
-        a = on ? -s_sc[o] : T(0);
-        if (!on) b = T(0);
+        if (two) {  // the lane's first separator, from the lane before
+            const T yp = __shfl_up(b, 1, W);
+            b1 = b;
+            b0 = j > 0 ? fma(a0, yp, b0) : b0;
+        } else {
+            b0 = b;
+        }
+        a0 = on ? -s_sc[o] : T(0);
+        a1 = on1 ? -s_sc[o1] : T(0);
+        if (!on) b0 = T(0);
+        if (!on1) b1 = T(0);
+        a = two ? a0 * a1 : a0;
+        b = two ? fma(a0, b1, b0) : b0;
         for (int d = 1; d < W; d <<= 1) {  // U z = y
             const T an = __shfl_down(a, d, W), bn = __shfl_down(b, d, W);
             if (j + d < W) {
                 b = fma(a, bn, b);
                 a *= an;
             }
+        }
+        if (two) {
+            const T zn = __shfl_down(b, 1, W);
+            if (on1) s_g[o1] = j + 1 < W ? fma(a1, zn, b1) : b1;
         }
         if (on) s_g[o] = b;
     } else if (seg == 0 && q.act) {

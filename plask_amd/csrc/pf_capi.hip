@@ -22,6 +22,7 @@
 #include "../../include/plask_fem.h"
 #include "fem_kernels.hpp"
 #include "batch_kernels.hpp"
+#include "batch_steps.hpp"
 #include "mg_kernels.hpp"
 
 using namespace pf;
@@ -387,9 +388,8 @@ static int part_lb(int m) {
 }
 
 static int part_threads(int P, int lb) {
-    int W = 1;
-    while (W < P - 1) W <<= 1;
-    return W <= 64 && W <= lb ? std::max(P, W) : P;
+    const int W = part_scan_lanes(P);
+    return W <= lb ? std::max(P, W) : P;
 }
 
 template <typename T>
@@ -3286,6 +3286,25 @@ int pf_time_apply(pf_ctx* ctx, int precision, int reps, double* seconds) {
 // ===========================================================================
 // Batched 2D Shockley solver (persistent kernel over a work queue)
 // ===========================================================================
+// Tables and launch shapes of the step-by-step batch solve
+struct BatchSteps {
+    bool ok = false;
+    BsArgs args{};
+    int levels = 0;  // levels outside the tail kernel, at most
+    struct Map {
+        BsBlock* p = nullptr;
+        int n = 0;
+    };
+    std::vector<Map> items, sweeps;  // per level outside the tail: operator items, sweep blocks
+    Map all_nodes0, elems, rows, line, factor, schur;
+    size_t sweep_lds = 0, up_lds = 0, tail_lds = 0, coarsen_lds = 0;
+    bool tail = false;
+    int* count = nullptr;   // pinned copy of args.count
+    hipGraphExec_t g_first = nullptr, g_loop = nullptr, g_iter = nullptr, g_start = nullptr, g_end = nullptr,
+                   g_cur = nullptr;
+    BatchParams prm{};
+};
+
 struct pf_batch {
     int device = 0;
     hipStream_t stream = nullptr;
@@ -3305,6 +3324,8 @@ struct pf_batch {
     unsigned int* hfin = nullptr;  // pinned: instances finished, read between launches
     // multigrid levels of all instances (pools described by BatchLevel)
     BatchMg mg{};
+    // all instances step by step (batch_steps.hpp), where the meshes allow it
+    BatchSteps steps;
     std::vector<long long> node_off;
     int tuned_block = 0, tuned_nwg = 0;
     std::vector<void*> allocs;
@@ -3329,9 +3350,170 @@ template <typename T> static int balloc(pf_batch* b, T** ptr, size_t count) {
     return PF_OK;
 }
 
+static void steps_drop(BatchSteps& S) {
+    for (hipGraphExec_t* g : {&S.g_first, &S.g_loop, &S.g_iter, &S.g_start, &S.g_end, &S.g_cur}) {
+        if (*g) hipGraphExecDestroy(*g);
+        *g = nullptr;
+    }
+}
+
 __global__ void k_copy_d(long long n, const double* __restrict__ a, double* __restrict__ b) {
     for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x)
         b[i] = a[i];
+}
+
+// Tables of the step-by-step solve: one entry per (instance, level) and the block lists of every
+// kind of launch, largest instances first.  Meshes whose lines have more segments than the
+// separator scan takes (n1 > 1032; the walk of one thread per column would be the chain of
+// latencies this solve avoids) or whose element rows do not fit k_bs_coarsen's LDS (n0 > 2049)
+// stay with the persistent kernel.
+static int steps_build(pf_batch* b, const std::vector<BatchInst>& inst, const std::vector<BatchLevel>& levs,
+                       const std::vector<int>& order, const std::vector<uint64_t>& mask,
+                       const std::vector<uint64_t>& lmask) {
+    BatchSteps& S = b->steps;
+    const int ninst = b->ninst;
+    long long widest = 0;
+    for (const BatchInst& I : inst) {
+        const int P = (I.n1 + BS_M - 1) / BS_M;
+        if (P > 1 && !part_scan_lanes(P)) return PF_OK;
+        if ((long long)I.n0 * I.n1 >= (1LL << 30)) return PF_OK;
+        widest = std::max<long long>(widest, I.n0);
+    }
+    S.coarsen_lds = sizeof(double) * 4 * (size_t)(widest - 1);
+    if (S.coarsen_lds > 65536) return PF_OK;
+    std::vector<BsLevel> tab;
+    std::vector<int> lev0(ninst), tail(ninst);
+    std::vector<unsigned char> fixed[2];  // of level 0, of the coarse levels
+    long long schur = 0, nelem = 0;
+    size_t tail_lds = 0;
+    for (int q = 0; q < ninst; ++q) {
+        const BatchInst& I = inst[q];
+        lev0[q] = (int)tab.size();
+        for (int l = 0; l <= I.nlev; ++l) {
+            BsLevel L{};
+            L.n0 = l ? levs[I.lev_off + l - 1].n0 : I.n0;
+            L.n1 = I.n1;
+            L.P = (I.n1 + BS_M - 1) / BS_M;
+            L.CB = std::max(1, std::min(std::min(L.n0, BS_T - 2), BS_T / std::max(L.P, part_scan_lanes(L.P))));  // k_bs_up: 2 more
+            L.node = l ? levs[I.lev_off + l - 1].node_off : I.node_off;
+            L.elem = l ? levs[I.lev_off + l - 1].elem_off : I.elem_off;
+            L.mask = l ? levs[I.lev_off + l - 1].mask_off : I.node_off;
+            L.h0 = l ? levs[I.lev_off + l - 1].h0_off : I.h0_off;
+            L.cx = l < I.nlev ? levs[I.lev_off + l].cx_off : 0;
+            L.mx = l < I.nlev ? levs[I.lev_off + l].mx_off : 0;
+            L.schur = schur;
+            schur += 3LL * std::max(L.P - 1, 1) * L.n0;
+            if (l) nelem = std::max(nelem, L.elem + (long long)(L.n0 - 1) * (L.n1 - 1));
+            const std::vector<uint64_t>& mk = l ? lmask : mask;
+            std::vector<unsigned char>& fx = fixed[l > 0];
+            L.seg = (long long)fx.size();
+            fx.resize(fx.size() + (size_t)L.P * L.n0, 0);
+            for (int k = 0; k < L.n1; ++k)
+                for (int c = 0; c < L.n0; ++c) {
+                    const long long bit = L.mask + (long long)k * L.n0 + c;
+                    if ((mk[bit >> 6] >> (bit & 63)) & 1ull)
+                        fx[L.seg + (size_t)(k / BS_M) * L.n0 + c] |= (unsigned char)(1u << (k % BS_M));
+                }
+            S.sweep_lds = std::max(S.sweep_lds, sizeof(double) * (size_t)part_lds_values(L.P, L.CB, BS_T));
+            S.up_lds = std::max(S.up_lds, sizeof(double) * (size_t)bs_up_lds(L.n1, L.P, L.CB));
+            tab.push_back(L);
+        }
+        tail[q] = I.nlev + 1;
+        long long nodes = 0;
+        for (int l = I.nlev; l >= 1; --l) {
+            const BsLevel& L = tab[lev0[q] + l];
+            nodes += (long long)L.n0 * L.n1;
+            if (!bs_tail_fits(L.n0, L.n1, L.P, nodes)) break;
+            tail[q] = l;
+            tail_lds = std::max(tail_lds, sizeof(double) * (size_t)(nodes + part_lds_values(L.P, L.n0, BS_TAIL)));
+        }
+        if (tail[q] <= I.nlev) S.tail = true;
+        S.levels = std::max(S.levels, std::min(tail[q], I.nlev + 1));
+    }
+    S.tail_lds = tail_lds;
+    // rows per operator item: long marches reuse the node window, short ones give a small batch
+    // enough waves
+    S.args.rows = b->N >= 4000000 ? 16 : b->N >= 1000000 ? 8 : 4;
+    int rc;
+    auto put = [&](auto** dst, const auto& v) -> int {
+        using T = typename std::remove_reference<decltype(v[0])>::type;
+        typename std::remove_const<T>::type* d = nullptr;
+        if (int r = balloc(b, &d, v.size())) return r;
+        if (!v.empty()) BHIPCK(hipMemcpy(d, v.data(), sizeof(T) * v.size(), hipMemcpyHostToDevice));
+        *dst = d;
+        return PF_OK;
+    };
+    std::vector<int> nred(ninst, 1);  // most blocks of an instance in a reducing launch
+    auto make = [&](BatchSteps::Map& m, auto&& blocks, bool red) -> int {
+        std::vector<BsBlock> v;
+        for (int q : order)
+            for (int l = 0; l <= inst[q].nlev; ++l) {
+                const long long nb = blocks(q, l);
+                for (long long k = 0; k < nb; ++k) v.push_back(BsBlock{q, l, (int)k, (int)nb});
+                if (red) nred[q] = std::max<int>(nred[q], (int)nb);
+            }
+        m.n = (int)v.size();
+        return v.empty() ? PF_OK : put(&m.p, v);
+    };
+    auto lv = [&](int q, int l) -> const BsLevel& { return tab[lev0[q] + l]; };
+    auto up = [](long long n, long long k) { return (n + k - 1) / k; };
+    S.items.resize(S.levels);
+    S.sweeps.resize(S.levels);
+    for (int f = 0; f < S.levels; ++f) {
+        auto on = [&](int q, int l) { return l == f && l < std::min(tail[q], inst[q].nlev + 1); };
+        if ((rc = make(S.items[f], [&](int q, int l) {
+                 return on(q, l) ? up(up(lv(q, l).n1, S.args.rows) * lv(q, l).n0, 256) : 0; }, f == 0)) ||
+            (rc = make(S.sweeps[f], [&](int q, int l) { return on(q, l) ? up(lv(q, l).n0, lv(q, l).CB) : 0; }, f == 0)))
+            return rc;
+    }
+    auto nodes = [&](int q, int l) { return up((long long)lv(q, l).n0 * lv(q, l).n1, 256); };
+    if ((rc = make(S.all_nodes0, [&](int q, int l) { return l ? 0 : nodes(q, l); }, false)) ||
+        (rc = make(S.elems, [&](int q, int l) {
+             return l ? 0 : up((long long)(lv(q, l).n0 - 1) * (lv(q, l).n1 - 1), 256); }, true)) ||
+        (rc = make(S.rows, [&](int q, int l) { return l ? 0LL : (long long)(lv(q, l).n1 - 1); }, false)) ||
+        (rc = make(S.line, nodes, false)) ||
+        (rc = make(S.factor, [&](int q, int l) { return up((long long)lv(q, l).P * lv(q, l).n0, 256); }, false)) ||
+        (rc = make(S.schur, [&](int q, int l) { return up(lv(q, l).n0, 64); }, false)))
+        return rc;
+    std::vector<long long> part(ninst);
+    long long npart = 0;
+    for (int q = 0; q < ninst; ++q) {
+        part[q] = npart;
+        npart += 2LL * nred[q];
+    }
+    BsArgs& A = S.args;
+    BsLevel* dl = nullptr;
+    int *dl0 = nullptr, *dt = nullptr;
+    long long* dp = nullptr;
+    if ((rc = put(&dl, tab)) || (rc = put(&dl0, lev0)) || (rc = put(&dt, tail)) || (rc = put(&dp, part)) ||
+        (rc = balloc(b, &A.schur, schur)) || (rc = balloc(b, &A.partials, npart)) || (rc = balloc(b, &A.st, ninst)) ||
+        (rc = balloc(b, &A.PB, b->N)) || (rc = balloc(b, &A.count, 2)))
+        return rc;
+    unsigned char* dfx[2] = {nullptr, nullptr};
+    double *ea[2], *eb[2];
+    for (int c = 0; c < 2; ++c)
+        if ((rc = put(&dfx[c], fixed[c])) || (rc = balloc(b, &ea[c], c ? nelem : b->E)) ||
+            (rc = balloc(b, &eb[c], c ? nelem : b->E)))
+            return rc;
+    BHIPCK(hipHostMalloc((void**)&S.count, 2 * sizeof(int), hipHostMallocDefault));
+    A.inst = b->dinst;
+    A.lev = dl;
+    A.lev0 = dl0;
+    A.tail = dt;
+    A.part = dp;
+    A.pool[0] = BsPool{b->r, b->z, b->q, b->la, b->lw, b->lc, b->kh, b->kv, ea[0], eb[0], b->h0, b->rm, b->dmask, dfx[0]};
+    A.pool[1] = BsPool{b->mg.b, b->mg.x, b->mg.r, b->mg.la, b->mg.lw, b->mg.lc, b->mg.kh, b->mg.kv, ea[1], eb[1],
+                       b->mg.h0, b->mg.rm, b->mg.mask, dfx[1]};
+    A.h1 = b->h1;
+    A.cx = b->mg.cx;
+    A.mx = b->mg.mx;
+    A.wx = b->mg.wx;
+    A.X = b->x;
+    A.PA = b->p;
+    A.cur = b->cur;
+    A.stats = b->dstats;
+    S.ok = true;
+    return PF_OK;
 }
 
 extern "C" {
@@ -3364,6 +3546,8 @@ void pf_batch_destroy(pf_batch* b) {
     hipStreamSynchronize(b->stream);
     if (b->graph) hipGraphExecDestroy(b->graph);
     if (b->graph_init) hipGraphExecDestroy(b->graph_init);
+    steps_drop(b->steps);
+    if (b->steps.count) hipHostFree(b->steps.count);
     for (void* p : b->allocs) hipFree(p);
     if (b->hfin) hipHostFree(b->hfin);
     hipStreamDestroy(b->stream);
@@ -3561,7 +3745,7 @@ int pf_batch_set(pf_batch* b, int ninst, int cylindrical, const int32_t* n0, con
     BHIPCK(hipMemcpy(b->kv0, sv, sizeof(double) * E, hipMemcpyHostToDevice));
     BHIPCK(hipMemcpy(b->dmask, mask.data(), sizeof(uint64_t) * mask.size(), hipMemcpyHostToDevice));
     BHIPCK(hipMemcpy(b->x0, x0.data(), sizeof(double) * N, hipMemcpyHostToDevice));
-    return PF_OK;
+    return steps_build(b, inst, levs, order, mask, lmask);
 }
 
 }  // extern "C"
@@ -3621,8 +3805,12 @@ template <typename F> static int batch_capture(pf_batch* b, hipGraphExec_t* exec
 // reads the number of finished instances and reports it through `progress`.  Every
 // launch advances each unfinished instance by at least one loop, so at most
 // ceil(maxloops / loop_budget) launches run.
+static int steps_run(pf_batch* b, const BatchParams& prm, double* seconds, void (*progress)(int, int, int, double, void*),
+                     void* user);
+
 static int batch_run(pf_batch* b, int block, int nwg, const BatchParams& prm, double* seconds,
                      void (*progress)(int, int, int, double, void*), void* user) {
+    if (prm.precond == 3 && b->steps.ok) return steps_run(b, prm, seconds, progress, user);
     int rc;
     if (b->graphs) {
         if (!b->graph_init && (rc = batch_capture(b, &b->graph_init, [&] { batch_launch_init(b); }))) return rc;
@@ -3670,6 +3858,151 @@ static int batch_run(pf_batch* b, int block, int nwg, const BatchParams& prm, do
     return PF_OK;
 }
 
+// The step-by-step solve (batch_steps.hpp).  Launches of one Picard loop:
+static void steps_vcycle(pf_batch* b, bool start) {
+    BatchSteps& S = b->steps;
+    hipStream_t st = b->stream;
+    auto sweep = [&](auto kernel, const BatchSteps::Map& m) {
+        if (m.n) hipLaunchKernelGGL(kernel, dim3(m.n), dim3(BS_T), S.sweep_lds, st, S.args, (const BsBlock*)m.p);
+    };
+    auto resid = [&](int l) {
+        if (S.items[l].n)
+            hipLaunchKernelGGL(k_bs_resid, dim3(S.items[l].n), dim3(256), 0, st, S.args, (const BsBlock*)S.items[l].p);
+    };
+    if (start) sweep(k_bs_sweep<BS_START>, S.sweeps[0]);
+    else sweep(k_bs_sweep<BS_UPD>, S.sweeps[0]);
+    for (int l = 0; l < S.levels; ++l) {
+        resid(l);
+        if (l + 1 < S.levels) sweep(k_bs_sweep<BS_DOWN>, S.sweeps[l + 1]);
+    }
+    if (S.tail) hipLaunchKernelGGL(k_bs_tail, dim3(b->ninst), dim3(BS_TAIL), S.tail_lds, st, S.args, b->ninst);
+    for (int l = S.levels - 1; l >= 0; --l) {
+        const BatchSteps::Map& m = S.sweeps[l];
+        if (m.n) hipLaunchKernelGGL(k_bs_up, dim3(m.n), dim3(BS_T), S.up_lds, st, S.args, (const BsBlock*)m.p);
+    }
+}
+
+static void steps_count(pf_batch* b) {
+    BatchSteps& S = b->steps;
+    hipLaunchKernelGGL(k_bs_count, dim3(1), dim3(256), 0, b->stream, S.args, b->ninst);
+}
+// instances iterating and ended, after what has been launched so far
+static int steps_read(pf_batch* b) {
+    BHIPCK(hipMemcpyAsync(b->steps.count, b->steps.args.count, 2 * sizeof(int), hipMemcpyDeviceToHost, b->stream));
+    BHIPCK(hipStreamSynchronize(b->stream));
+    return PF_OK;
+}
+
+template <int PHASE> static void steps_true(pf_batch* b) {
+    BatchSteps& S = b->steps;
+    hipLaunchKernelGGL(k_bs_true<PHASE>, dim3(S.items[0].n), dim3(256), 0, b->stream, S.args, (const BsBlock*)S.items[0].p);
+}
+
+// one graph per phase, captured on its first use with these parameters
+template <typename F> static int steps_phase(pf_batch* b, hipGraphExec_t* g, F&& launches) {
+    if (!b->graphs) {
+        launches();
+        BHIPCK(hipGetLastError());
+        return PF_OK;
+    }
+    if (!*g)
+        if (int rc = batch_capture(b, g, launches)) return rc;
+    BHIPCK(hipGraphLaunch(*g, b->stream));
+    return PF_OK;
+}
+
+static int steps_run(pf_batch* b, const BatchParams& prm, double* seconds, void (*progress)(int, int, int, double, void*),
+                     void* user) {
+    BatchSteps& S = b->steps;
+    if (!same_prm(S.prm, prm)) {
+        steps_drop(S);
+        S.prm = prm;
+        S.args.coarse_sweeps = prm.coarse_sweeps;
+        S.args.maxit = prm.maxit;
+        S.args.maxloops = prm.maxloops;
+        S.args.stable = prm.stable;
+        S.args.omega = prm.omega;
+        S.args.rtol = prm.rtol;
+        S.args.maxerr = prm.maxerr;
+    }
+    hipStream_t st = b->stream;
+    auto on = [&](auto kernel, const BatchSteps::Map& m, int threads, size_t lds = 0) {
+        if (m.n) hipLaunchKernelGGL(kernel, dim3(m.n), dim3(threads), lds, st, S.args, (const BsBlock*)m.p);
+    };
+    const auto t0 = std::chrono::steady_clock::now();
+    int rc;
+    hipEvent_t e0, e1;
+    BHIPCK(hipEventCreate(&e0));
+    BHIPCK(hipEventCreate(&e1));
+    BHIPCK(hipEventRecord(e0, st));
+    if ((rc = steps_phase(b, &S.g_first, [&] {
+             batch_launch_init(b);
+             hipLaunchKernelGGL(k_bs_reset, dim3((b->ninst + 255) / 256), dim3(256), 0, st, S.args, b->ninst);
+             steps_true<0>(b);
+         })))
+        return rc;
+    int launches = 0;
+    for (int loop = 0; loop < prm.maxloops; ++loop) {
+        if ((rc = steps_phase(b, &S.g_loop, [&] {
+                 hipLaunchKernelGGL(k_bs_junction, dim3(b->ninst), dim3(256), 0, st, S.args);
+                 on(k_bs_coarsen, S.rows, 64, S.coarsen_lds);
+                 on(k_bs_line, S.line, 256);
+                 on(k_bs_factor, S.factor, 256);
+                 on(k_bs_schur, S.schur, 64);
+                 steps_true<1>(b);
+                 steps_vcycle(b, true);
+             })))
+            return rc;
+        // CG runs (a second one for the instances whose true residual asks for it)
+        for (;;) {
+            do {
+                if ((rc = steps_phase(b, &S.g_iter, [&] {
+                         for (int c = 0; c < 4; ++c) {
+                             on(k_bs_apply, S.items[0], 256);
+                             steps_vcycle(b, false);
+                         }
+                         steps_count(b);
+                     })))
+                    return rc;
+                if ((rc = steps_read(b))) return rc;
+            } while (S.count[0] > 0);
+            if ((rc = steps_phase(b, &S.g_end, [&] {
+                     on(k_bs_fixup, S.all_nodes0, 256);
+                     steps_true<2>(b);
+                     steps_count(b);
+                 })))
+                return rc;
+            if ((rc = steps_read(b))) return rc;
+            if (S.count[0] == 0) break;
+            if ((rc = steps_phase(b, &S.g_start, [&] { steps_vcycle(b, true); }))) return rc;
+        }
+        if ((rc = steps_phase(b, &S.g_cur, [&] {
+                 on(k_bs_currents, S.elems, 256);
+                 steps_count(b);
+             })))
+            return rc;
+        if ((rc = steps_read(b))) return rc;
+        const bool end = S.count[1] == b->ninst || loop + 1 == prm.maxloops;
+        if (end || (prm.loop_budget > 0 && (loop + 1) % prm.loop_budget == 0)) {
+            ++launches;
+            if (progress)
+                progress(launches, S.count[1], b->ninst,
+                         std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count(), user);
+        }
+        if (end) break;
+    }
+    hipLaunchKernelGGL(k_bs_total, dim3(b->ninst), dim3(256), 0, st, S.args);
+    BHIPCK(hipGetLastError());
+    BHIPCK(hipEventRecord(e1, st));
+    BHIPCK(hipEventSynchronize(e1));
+    float ms = 0.f;
+    hipEventElapsedTime(&ms, e0, e1);
+    hipEventDestroy(e0);
+    hipEventDestroy(e1);
+    if (seconds) *seconds = 1e-3 * ms;
+    return PF_OK;
+}
+
 extern "C" {
 
 int pf_batch_autotune(pf_batch* b, const pf_batch_opts* o, int* best_block, int* best_nwg, double* best_seconds) {
@@ -3691,8 +4024,10 @@ int pf_batch_autotune(pf_batch* b, const pf_batch_opts* o, int* best_block, int*
     const int mult[2] = {1, 2};
     double best = 1e300;
     int bb = 1024, bn = props_cu;
-    for (int bi = 0; bi < 3; ++bi)
-        for (int mi = 0; mi < 2; ++mi) {
+    // the step-by-step solve has no such choice: one run gives its time
+    const bool steps = prm.precond == 3 && b->steps.ok;
+    for (int bi = steps ? 2 : 0; bi < 3; ++bi)
+        for (int mi = 0; mi < (steps ? 1 : 2); ++mi) {
             int nwg = std::min(b->ninst, props_cu * mult[mi]);
             double t = 0.;
             int rc = batch_run(b, blocks[bi], nwg, prm, &t, o->progress, o->progress_user);

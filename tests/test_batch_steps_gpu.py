@@ -1,0 +1,85 @@
+"""Batches whose instances advance together (multigrid preconditioner), at the sizes where the
+launch shapes change: meshes without coarse levels, rows and columns around a segment and a
+block, one and two separators per scan lane, lines too long for the scan (persistent kernel)."""
+import numpy as np
+import pytest
+
+import oracle as O
+from plask_amd.batch import PROGRESS, ShockleyBatch
+
+pytestmark = pytest.mark.gpu
+
+
+def _instance(n0, n1, seed, junction=True):
+    rng = np.random.default_rng(seed)
+    r = np.r_[0.0, np.cumsum(rng.uniform(0.5, 1.5, n0 - 1))]
+    z = np.r_[0.0, np.cumsum(rng.uniform(0.05, 0.15, n1 - 1))]
+    E0 = n0 - 1
+    sig = np.exp(rng.uniform(np.log(10.0), np.log(1e3), n1 - 1))
+    sh, sv = np.repeat(sig, E0), np.repeat(sig, E0)
+    jlo = (n1 - 1) // 2
+    jhi = jlo + 1 if junction else jlo
+    sh[jlo * E0:jhi * E0], sv[jlo * E0:jhi * E0] = 0.0, 5.0
+    # contact over the top row but its last node, the whole bottom row, one fixed node on the side
+    top = (n1 - 1) * n0 + np.arange(n0 - 1)
+    side = [(n1 // 2) * n0 + n0 - 1] if n1 > 4 else []
+    dn = np.r_[np.arange(n0), top, side].astype(np.int64)
+    dv = np.r_[np.zeros(n0), np.full(len(top), 1.5), np.full(len(side), 0.4)]
+    return dict(axes=[r, z], sh=sh, sv=sv, dir_nodes=dn, dir_vals=dv, jlo=jlo, jhi=jhi, beta=8.0, js=1.0)
+
+
+def _oracle(p, loops):
+    r, z = p["axes"]
+    g = O.Grid([r, z], cyl=True)
+    E0 = len(r) - 1
+    elems = np.arange(p["jlo"] * E0, p["jhi"] * E0)
+    J = []
+    if len(elems):
+        bot = [[e % E0 + p["jlo"] * len(r), e % E0 + 1 + p["jlo"] * len(r)] for e in elems]
+        top = [[e % E0 + p["jhi"] * len(r), e % E0 + 1 + p["jhi"] * len(r)] for e in elems]
+        J = [dict(elems=elems, bottom=bot, top=top, height=z[p["jhi"]] - z[p["jlo"]], beta=p["beta"], js=p["js"])]
+    return O.electrical_compute(g, p["sh"].copy(), p["sv"].copy(), p["dir_nodes"], p["dir_vals"], J, loops, maxerr=0.0)
+
+
+@pytest.mark.parametrize("sizes", [
+    [(2, 2), (2, 3), (3, 8), (3, 9), (2, 40)],                    # no coarse level
+    [(4, 7), (4, 8), (5, 17), (9, 16), (33, 64), (65, 65)],       # segments of axis 1, tails
+    [(300, 8), (513, 5), (600, 9), (129, 33), (30, 3)],           # widest sweep blocks
+    [(7, 512), (12, 513), (5, 521), (20, 528), (3, 1032)],        # 63 to 128 separators
+    [(20, 130), (4, 1033), (2, 2)],                               # a line too long for the scan
+])
+def test_steps_match_oracle(sizes):
+    """CG stops at 1e-13 of each loop's start residual, so the potentials agree with the direct
+    solve to the conditioning of the systems times that, as in the other batch tests: 1e-8."""
+    insts = [_instance(n0, n1, 10 * k + n1, junction=(k % 3 != 1 and n1 > 2)) for k, (n0, n1) in enumerate(sizes)]
+    b = ShockleyBatch(insts)
+    print("batch steps", sizes, flush=True)
+    for _ in range(2):  # the second solve replays the graphs on the state the first one left
+        V, stats, _t = b.solve(maxloops=3, maxerr=1e-30, rtol=1e-13, precond=3)
+        for size, p, v, s in zip(sizes, insts, V, stats):
+            Vr, loops = _oracle(p, 3)[0], _oracle(p, 3)[4]
+            assert s["status"] in (0, 2) and s["loops"] <= 3, (size, s)
+            assert np.abs(v - Vr).max() <= 1e-8 * np.abs(Vr).max(), (size, np.abs(v - Vr).max(), s)
+
+
+def test_steps_progress_and_options():
+    """progress comes after every loop_budget loops; loop and iteration limits end the loop with
+    the status of the persistent kernel; block and nwg choose nothing here."""
+    insts = [_instance(20 + 9 * k, 40 + 11 * k, k) for k in range(4)]
+    b = ShockleyBatch(insts)
+    seen = []
+    o = b.opts(maxloops=5, maxerr=1e-30, rtol=1e-12, loop_budget=2)
+    o.progress = PROGRESS(lambda *a: seen.append(a[:3]))
+    b.opts = lambda **kw: o
+    V, stats, _t = b.solve()
+    del b.opts
+    assert [s[0] for s in seen] == [1, 2, 3] and seen[-1][1:] == (4, 4), seen
+    V2, stats2, _t = b.solve(maxloops=5, maxerr=1e-30, rtol=1e-12, block=256, nwg=3)
+    for a, c in zip(V, V2):
+        assert np.array_equal(a, c)
+    # iteration limit in every loop, error limit never met and met at once
+    for maxerr in (1e-30, 1e9):
+        kw = dict(maxloops=5, maxit=2, maxerr=maxerr, rtol=1e-12)
+        st, sp = b.solve(precond=3, **kw)[1], b.solve(precond=2, **kw)[1]
+        for a, c in zip(st, sp):
+            assert (a["status"], a["loops"], a["iters"]) == (c["status"], c["loops"], c["iters"]), (a, c)
