@@ -1,0 +1,62 @@
+"""Operator, line preconditioner and V-cycle at the sizes where the default launch shapes and the
+separator scan change: few and many rows per tile, one plane per block, 24 segments in a scan of
+32 lanes, one and two separators per lane, lines too long for the scan."""
+import numpy as np
+import pytest
+
+import oracle as O
+from oracle import multigrid as MG
+from plask_amd.fem import PF_FP32_RELIABLE, PF_FP64, PRECOND_LINE, PRECOND_MG, FemContext
+
+pytestmark = pytest.mark.gpu
+
+
+def _problem(shape, cyl=False):
+    rng = np.random.default_rng(sum(shape))
+    axes = [np.cumsum(np.r_[0.0, rng.uniform(0.05, 2.0, n - 1)]) for n in shape]
+    g = O.Grid(axes, cyl=cyl)
+    kh, kv = rng.uniform(0.5, 150.0, g.nelems), rng.uniform(0.5, 150.0, g.nelems)
+    plane = g.nnodes // shape[-1]
+    dn = np.r_[np.arange(plane), rng.choice(np.arange(plane, g.nnodes), 3, replace=False)].astype(np.int64)
+    c = FemContext()
+    c.set_grid(axes, cylindrical=cyl)
+    c.set_coeffs(kh, kv)
+    c.set_source(np.zeros(g.nelems))
+    c.set_dirichlet(dn, np.full(len(dn), 300.0))
+    return g, axes, kh, kv, dn, c
+
+
+@pytest.mark.parametrize("shape", [(2, 2, 2), (17, 17, 5), (25, 19, 37), (128, 3, 9), (300, 2, 3), (65, 65, 8),
+                                   (2, 3), (33, 63), (33, 64), (33, 257), (700, 65)])
+def test_default_launch_shapes_apply(shape):
+    """y = A x (FP64) against the oracle's element sums: rounding of 27 products, 1e-13 of the largest."""
+    g, axes, kh, kv, dn, c = _problem(shape)
+    print("launch shapes apply", shape, flush=True)
+    mask = np.zeros(g.nnodes, np.uint8)
+    mask[dn] = 1
+    x = np.random.default_rng(1).uniform(-1, 1, g.nnodes)
+    ref = O.apply(g, 0, kh, kv, mask, x)
+    y = c.apply(x)
+    assert np.abs(y - ref).max() <= 1e-13 * np.abs(ref).max()
+    c.close()
+
+
+@pytest.mark.parametrize("shape", [(3, 3, 192), (5, 4, 520), (4, 3, 521), (3, 4, 1024), (5, 520), (5, 521), (4, 1032),
+                                   (4, 1033)])
+def test_long_lines_vcycle(shape):
+    """One V-cycle against the CPU statement of it (its line solves are direct): 1e-10 in FP64,
+    norm-wise 1e-3 with FP32 line solves, as in the other V-cycle tests."""
+    g, axes, kh, kv, dn, c = _problem(shape)
+    print("long lines", shape, flush=True)
+    r = np.random.default_rng(2).uniform(-1, 1, g.nnodes)
+    r[dn] = 0.0
+    z_ref = MG.VCycle(axes, kh, kv, dn).apply(r)
+    z = c.precond_apply(r, PF_FP64, PRECOND_MG)
+    assert np.abs(z - z_ref).max() <= 1e-10 * np.abs(z_ref).max()
+    z32 = c.precond_apply(r, PF_FP32_RELIABLE, PRECOND_MG)
+    assert np.linalg.norm(z32 - z_ref) <= 1e-3 * np.linalg.norm(z_ref)
+    c.set_line_segment(-1)
+    zl = c.precond_apply(r, PF_FP64, PRECOND_LINE)
+    c.set_line_segment(0)
+    assert np.abs(c.precond_apply(r, PF_FP64, PRECOND_LINE) - zl).max() <= 1e-10 * np.abs(zl).max()
+    c.close()
