@@ -252,7 +252,7 @@ int pf_kernel_times(pf_ctx* ctx, double* seconds, int64_t* counts, int n);
 
 /* Launch shape of the operator kernels (for tuning): 3D rows = thread rows per block
  * (rows * n0 <= 1024, one of them a halo row), planes = planes per block along axis 2;
- * 2D planes = rows of axis 1 per block. */
+ * 2D planes = rows of axis 1 per thread. */
 int pf_set_launch(pf_ctx* ctx, int rows, int planes);
 
 /* Line preconditioner schedule (the preconditioner itself, the exact tridiagonal

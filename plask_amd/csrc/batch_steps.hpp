@@ -346,7 +346,7 @@ __global__ __launch_bounds__(BS_T, 4) void k_bs_sweep(BsArgs A, const BsBlock* _
     const PartPos q = part_pos(L.n0, L.n1, L.P, L.CB, plane, BS_M, B.local);
     double* b = P.b + L.node;
     double* r = P.r + L.node;
-    double rv[BS_M], av[BS_M], wv[BS_M], cv[BS_M];
+    double rv[BS_M], qv[BS_M], av[BS_M], wv[BS_M], cv[BS_M], sv[3];
     double rr = 0.;
     if (MODE == BS_DOWN) {
         const BsLevel F = LV[-1];
@@ -370,25 +370,25 @@ __global__ __launch_bounds__(BS_T, 4) void k_bs_sweep(BsArgs A, const BsBlock* _
             }
         }
     } else {
-        const double alpha = MODE == BS_UPD ? S.alpha : 0.;
+        part_load<double, BS_M>(q, plane, b, rv);
+        if (MODE == BS_UPD) {
+            const double alpha = S.alpha;
+            part_load<double, BS_M>(q, plane, r, qv);  // level 0: q = A p lies in r
+            part_factors<double, BS_M>(q, L.P, L.n0, plane, P.la + L.node, P.lw + L.node, P.lc + L.node, A.schur + L.schur,
+                                       av, wv, cv, sv);
 #pragma unroll
-        for (int u = 0; u < BS_M; ++u) {
-            rv[u] = 0.;
-            if (u < q.len) {
-                const long long node = q.base + (long long)u * plane;
-                rv[u] = b[node];
-                if (MODE == BS_UPD) {
-                    rv[u] -= alpha * r[node];  // level 0: q = A p lies in r
-                    b[node] = rv[u];
-                    rr += rv[u] * rv[u];
-                }
+            for (int u = 0; u < BS_M; ++u) {
+                rv[u] -= alpha * qv[u];
+                rr += rv[u] * rv[u];
+                if (u < q.len) b[q.base + (long long)u * plane] = rv[u];
             }
         }
     }
-    part_factors<double, BS_M>(q, plane, P.la + L.node, P.lw + L.node, P.lc + L.node, av, wv, cv);
+    if (MODE != BS_UPD)
+        part_factors<double, BS_M>(q, L.P, L.n0, plane, P.la + L.node, P.lw + L.node, P.lc + L.node, A.schur + L.schur, av,
+                                   wv, cv, sv);
     double zv[BS_M];
-    part_solve<double, BS_M>(q, L.P, L.CB, L.n0, A.schur + L.schur, reinterpret_cast<double*>(part_smem), rv, av, wv, cv,
-                             zv);
+    part_solve<double, BS_M>(q, L.P, L.CB, reinterpret_cast<double*>(part_smem), rv, av, wv, cv, sv, zv);
 #pragma unroll
     for (int u = 0; u < BS_M; ++u)
         if (u < q.len) r[q.base + (long long)u * plane] = A.omega * zv[u];
@@ -421,13 +421,15 @@ inline bool bs_tail_fits(int n0, int n1, int P, long long nodes) {  // nodes: of
 // What a thread keeps of its segment on a level: line factors, element coefficients of the
 // layers around it on both sides (0 where there is none), Dirichlet nodes.
 struct BsSegment {
-    double av[BS_M], wv[BS_M], cv[BS_M];
+    double av[BS_M], wv[BS_M], cv[BS_M], sv[3];
     double c[BS_M + 1][4];
     unsigned fixed;
 };
 
-__device__ __forceinline__ void bs_segment(const BsLevel& L, const BsPool& P, const PartPos& q, BsSegment& G) {
-    part_factors<double, BS_M>(q, L.n0, P.la + L.node, P.lw + L.node, P.lc + L.node, G.av, G.wv, G.cv);
+__device__ __forceinline__ void bs_segment(const BsLevel& L, const BsPool& P, const double* schur, const PartPos& q,
+                                           BsSegment& G) {
+    part_factors<double, BS_M>(q, L.P, L.n0, L.n0, P.la + L.node, P.lw + L.node, P.lc + L.node, schur + L.schur, G.av, G.wv,
+                               G.cv, G.sv);
     G.fixed = q.act ? P.fixed[L.seg + q.seg * L.n0 + q.col] : 0u;
     const int i = q.act ? q.col : 0, k0 = q.act ? q.seg * BS_M : 0;
     const int eL = max(i - 1, 0), eR = min(i, L.n0 - 2);
@@ -506,7 +508,7 @@ __global__ __launch_bounds__(BS_T, 2) void k_bs_up(BsArgs A, const BsBlock* __re
     double* xt = ps + part_lds_values(L.P, L.CB, BS_T);
     // the segment's own data travels while the tile is staged
     BsSegment G;
-    bs_segment(L, P, q, G);
+    bs_segment(L, P, A.schur, q, G);
     double rv[BS_M], bv[BS_M], zv[BS_M];
 #pragma unroll
     for (int u = 0; u < BS_M; ++u) bv[u] = u < q.len ? P.b[L.node + q.base + (long long)u * L.n0] : 0.;
@@ -546,7 +548,7 @@ __global__ __launch_bounds__(BS_T, 2) void k_bs_up(BsArgs A, const BsBlock* __re
 #pragma unroll
     for (int u = 0; u < BS_M; ++u) rv[u] = bv[u];
     bs_lds_residual(L, xt, HX, pad, q.cl, q.cl + 1, q.cl + 2, q, G, rv);
-    part_solve<double, BS_M>(q, L.P, L.CB, L.n0, A.schur + L.schur, ps, rv, G.av, G.wv, G.cv, zv);
+    part_solve<double, BS_M>(q, L.P, L.CB, ps, rv, G.av, G.wv, G.cv, G.sv, zv);
     double rz = 0.;
 #pragma unroll
     for (int u = 0; u < BS_M; ++u) {
@@ -586,7 +588,7 @@ __global__ __launch_bounds__(BS_TAIL) void k_bs_tail(BsArgs A, int ninst) {
         const BsLevel L = LV[l], F = LV[l - 1];
         const PartPos q = pos(L);
         BsSegment G;
-        bs_segment(L, P, q, G);
+        bs_segment(L, P, A.schur, q, G);
         double* x = xs + (L.node - xnode0);
         double bv[BS_M], rv[BS_M], zv[BS_M];
         {
@@ -607,7 +609,7 @@ __global__ __launch_bounds__(BS_TAIL) void k_bs_tail(BsArgs A, int ninst) {
             }
         }
         __syncthreads();  // the finer level's residual is read
-        part_solve<double, BS_M>(q, L.P, L.n0, L.n0, A.schur + L.schur, ps, bv, G.av, G.wv, G.cv, zv);
+        part_solve<double, BS_M>(q, L.P, L.n0, ps, bv, G.av, G.wv, G.cv, G.sv, zv);
 #pragma unroll
         for (int u = 0; u < BS_M; ++u)
             if (u < q.len) x[q.base + (long long)u * L.n0] = A.omega * zv[u];
@@ -625,7 +627,7 @@ __global__ __launch_bounds__(BS_TAIL) void k_bs_tail(BsArgs A, int ninst) {
                 break;
             }
             __syncthreads();
-            part_solve<double, BS_M>(q, L.P, L.n0, L.n0, A.schur + L.schur, ps, rv, G.av, G.wv, G.cv, zv);
+            part_solve<double, BS_M>(q, L.P, L.n0, ps, rv, G.av, G.wv, G.cv, G.sv, zv);
 #pragma unroll
             for (int u = 0; u < BS_M; ++u)
                 if (u < q.len) x[q.base + (long long)u * L.n0] += A.omega * zv[u];
@@ -636,7 +638,7 @@ __global__ __launch_bounds__(BS_TAIL) void k_bs_tail(BsArgs A, int ninst) {
         const BsLevel L = LV[l], C = LV[l + 1];
         const PartPos q = pos(L);
         BsSegment G;
-        bs_segment(L, P, q, G);
+        bs_segment(L, P, A.schur, q, G);
         double rv[BS_M], zv[BS_M];
 #pragma unroll
         for (int u = 0; u < BS_M; ++u) rv[u] = u < q.len ? P.b[L.node + q.base + (long long)u * L.n0] : 0.;
@@ -653,7 +655,7 @@ __global__ __launch_bounds__(BS_TAIL) void k_bs_tail(BsArgs A, int ninst) {
             }
         __syncthreads();
         bs_lds_residual(L, x, L.n0, 0, max(q.col - 1, 0), q.col, min(q.col + 1, L.n0 - 1), q, G, rv);
-        part_solve<double, BS_M>(q, L.P, L.n0, L.n0, A.schur + L.schur, ps, rv, G.av, G.wv, G.cv, zv);
+        part_solve<double, BS_M>(q, L.P, L.n0, ps, rv, G.av, G.wv, G.cv, G.sv, zv);
 #pragma unroll
         for (int u = 0; u < BS_M; ++u)
             if (u < q.len) x[q.base + (long long)u * L.n0] += A.omega * zv[u];

@@ -90,6 +90,7 @@ template <typename T> struct Axes2 {
     int n0, n1;
     const T* hx;    // element sizes (um)
     const T* hy;
+    const T* rhy;   // 1 / hy
     const T* rmid;  // cylindrical: element mid radius, else nullptr
     const T* dsh = nullptr;
 };
@@ -174,6 +175,10 @@ __device__ bool grid_reduce(double (&v)[NV], double* __restrict__ partials, unsi
     if (tid == 0) __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     return tid == 0;
 }
+
+// Keeps the loads before it from being moved behind it (past a branch they do not depend on):
+// they are in flight while that branch waits.
+__device__ __forceinline__ void issue_loads() { asm volatile("" ::: "memory"); }
 
 // ---------------------------------------------------------------------------
 // 3D operator apply, z-marching.
@@ -713,137 +718,154 @@ __global__ __launch_bounds__(512) void k_apply3r(Axes3<T> g, int KR, int nb, con
 }
 
 // ---------------------------------------------------------------------------
-// 2D operator apply (Cartesian or cylindrical), marching along axis 1.
-// One block = the whole row (BX = n0 threads); thread tx owns element column tx
-// and node column tx.  Element matrix therm2d.cpp:216-228, x r_mid for
-// cylindrical geometry (therm2d.cpp:333,410-420; electr2d.cpp:206-231).
+// 2D operator apply (Cartesian or cylindrical): a thread marches KC rows of one column along
+// axis 1, neighbour columns and their elements read through the cache.  Element matrix
+// therm2d.cpp:216-228, x r_mid for cylindrical geometry (therm2d.cpp:333,410-420;
+// electr2d.cpp:206-231), in the sum / difference basis: of a layer with coefficients
+// a = kx' / 12 and b = ky' / 12, the row above gets S + D and the row below S - D.
+// Held by latency at the usual sizes (a 200 x 400 grid and its coarse levels are 0.4 to 16 MB):
+// no barriers, and the loads of the first U rows and of the two around them are issued before
+// the stop flag is waited for: the residuals of that solve's levels take 3.4 us and its fused
+// apply 8.5 us (a block per row, LDS and two barriers per row: 4.9 and 12.2 us).
 // ---------------------------------------------------------------------------
-template <typename T, int MODE, bool FUSEP, bool DOT>
-__global__ __launch_bounds__(1024) void k_apply2d(Axes2<T> g, int KC, const T* __restrict__ xin,
-                                                  const T* __restrict__ zin, const T* __restrict__ pin,
-                                                  T* __restrict__ pout, T* __restrict__ xsol, T* __restrict__ y,
-                                                  const T* __restrict__ F, const uint64_t* __restrict__ dmask,
-                                                  const T* __restrict__ kh, const T* __restrict__ kv,
-                                                  PcgState* __restrict__ st, double* __restrict__ partials) {
-    extern __shared__ unsigned char smem_raw[];
+template <typename T, int MODE, bool FUSEP, bool DOT, int U>
+__global__ __launch_bounds__(256) void k_apply2d(Axes2<T> g, int KC, const T* __restrict__ xin,
+                                                 const T* __restrict__ zin, const T* __restrict__ pin,
+                                                 T* __restrict__ pout, T* __restrict__ xsol, T* __restrict__ y,
+                                                 const T* __restrict__ F, const uint64_t* __restrict__ dmask,
+                                                 const T* __restrict__ kh, const T* __restrict__ kv,
+                                                 PcgState* __restrict__ st, double* __restrict__ partials) {
     const int n0 = g.n0, n1 = g.n1;
-    const int PX = n0 + 1;
-    T* xs = reinterpret_cast<T*>(smem_raw);  // [2][PX]
-    T* oc = xs + 2 * PX;                     // [2][PX], corner outputs at column tx+1
+    const int w = (int)(blockIdx.x * 256 + threadIdx.x);
+    const int chunk = w / n0, i = w - chunk * n0;
+    const bool live = (long long)chunk * KC < n1;
+    const int kb = live ? chunk * KC : 0, ke = live ? min(kb + KC, n1) : 0;
+    const int il = max(i - 1, 0), ir = min(i + 1, n0 - 1);
+    const int eL = max(i - 1, 0), eR = min(i, n0 - 2);
+    struct Row {
+        T z[3], p[3], x, f, ds;  // columns i - 1, i, i + 1
+        uint32_t d[3];
+    };
+    struct Layer {
+        T hl, hr, vl, vr, h, rh;
+    };
+    const uint32_t* dmask32 = reinterpret_cast<const uint32_t*>(dmask);
+    auto load_row = [&](int kk, Row& R) {
+        const long long o = (long long)min(max(kk, 0), n1 - 1) * n0;
+        const long long c[3] = {o + il, o + i, o + ir};
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+            if (FUSEP) {
+                R.z[q] = zin[c[q]];
+                R.p[q] = pin[c[q]];
+            } else {
+                R.z[q] = xin[c[q]];
+            }
+            if (MODE == MODE_OP || q == 1) R.d[q] = dmask32[c[q] >> 5] >> (c[q] & 31);
+        }
+        if (FUSEP) R.x = xsol[c[1]];
+        if (MODE != MODE_OP) R.f = F[c[1]];
+        R.ds = g.dsh ? g.dsh[c[1]] : T(0);
+    };
+    auto load_layer = [&](int e, Layer& L) {  // between rows e and e + 1
+        const int ec = min(max(e, 0), n1 - 2);
+        const long long o = (long long)ec * (n0 - 1);
+        L.hl = kh[o + eL];
+        L.hr = kh[o + eR];
+        L.vl = kv[o + eL];
+        L.vr = kv[o + eR];
+        L.h = g.hy[ec];
+        L.rh = g.rhy[ec];
+    };
+    Row Ra, Rb, R[U];
+    Layer Lb, L[U];
+    load_row(kb - 1, Ra);
+    load_row(kb, Rb);
+    load_layer(kb - 1, Lb);
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        load_row(kb + 1 + u, R[u]);
+        load_layer(kb + u, L[u]);
+    }
+    const T wl = g.hx[eL], wr = g.hx[eR], rl = g.rmid ? g.rmid[eL] : T(1), rr = g.rmid ? g.rmid[eR] : T(1);
+    issue_loads();
     if (FUSEP || DOT || MODE == MODE_RESG) {
         if (st->done) return;
     }
-    const int tx = threadIdx.x;
-    const bool nvalid = tx < n0;
-    const bool evalid = tx < n0 - 1;
-    const int kb = blockIdx.x * KC;
-    const int ke = min(kb + KC, n1);
-    double beta = 0.;
-    T alpha_prev = T(0);
+    T beta = T(0), alpha_prev = T(0);
     if (FUSEP) {
-        beta = (st->iters == 0) ? st->beta0 : st->rz / st->rz_prev;
+        beta = T((st->iters == 0) ? st->beta0 : st->rz / st->rz_prev);
         alpha_prev = T(st->alpha);
     }
-
-    T gxf = 0, gyf = 0;
-    if (evalid) {
-        T w = g.hx[tx];
-        T r = g.rmid ? g.rmid[tx] : T(1);
-        gxf = r / (T(12) * w);  // kx' / 12 = kx h r / (12 w)
-        gyf = r * w / T(12);    // ky' / 12 = ky w r / (12 h)
-    }
-    if (threadIdx.x < 2) {
-        xs[threadIdx.x * PX + n0] = T(0);
-        oc[threadIdx.x * PX] = T(0);
-    }
-    auto load_row = [&](int k, int buf, T& own, bool& d, bool store_p) {
-        T v = T(0);
-        d = false;
-        if (nvalid) {
-            long long node = (long long)k * n0 + tx;
-            if (FUSEP) {
-                const T po = pin[node];
-                v = zin[node] + T(beta) * po;
-                if (store_p) {
-                    pout[node] = v;
-                    xsol[node] += alpha_prev * po;
-                }
-            } else {
-                v = xin[node];
-            }
-            d = dbit(dmask, node);
-            xs[buf * PX + tx] = (MODE == MODE_OP && d) ? T(0) : v;
+    // kx' / 12 = kx h r / (12 w), ky' / 12 = ky w r / (12 h); no element left of column 0 and
+    // right of the last one
+    const T fl = i > 0 ? T(1) : T(0), fr = i < n0 - 1 ? T(1) : T(0);
+    const T gxl = fl * (rl / (T(12) * wl)), gyl = fl * (rl * wl / T(12));
+    const T gxr = fr * (rr / (T(12) * wr)), gyr = fr * (rr * wr / T(12));
+    // operand of a row (masked for MODE_OP) in the basis of the two element columns
+    auto operand = [&](const Row& r, T (&t)[4], T& own) {
+        T v[3];
+#pragma unroll
+        for (int q = 0; q < 3; ++q) v[q] = FUSEP ? r.z[q] + beta * r.p[q] : r.z[q];
+        own = v[1];
+        if (MODE == MODE_OP) {
+#pragma unroll
+            for (int q = 0; q < 3; ++q)
+                if (r.d[q] & 1u) v[q] = T(0);
         }
-        own = v;
+        t[0] = v[0] + v[1];
+        t[1] = v[1] - v[0];
+        t[2] = v[1] + v[2];
+        t[3] = v[1] - v[2];
     };
-    const int P0 = (kb > 0) ? kb - 1 : 0;
-    int buf = 0;
-    T own_cur, own_next = T(0);
-    bool dir_cur, dir_next = false;
-    __syncthreads();
-    load_row(P0, 0, own_cur, dir_cur, FUSEP && P0 >= kb);
-    __syncthreads();
-    T s_cur = T(0), d_cur = T(0);
-    if (nvalid) {
-        T v0 = xs[tx], v1 = xs[tx + 1];
-        s_cur = v0 + v1;
-        d_cur = v1 - v0;
-    }
-    T acc0 = T(0), acc1 = T(0);
+    auto layer = [&](int e, const Layer& c, const T (&lo)[4], const T (&up)[4], T& S, T& D) {
+        const T on = e >= 0 && e < n1 - 1 ? T(1) : T(0);
+        const T al = c.hl * (gxl * (on * c.h)), ar = c.hr * (gxr * (on * c.h));
+        const T bl = c.vl * (gyl * (on * c.rh)), br = c.vr * (gyr * (on * c.rh));
+        S = (up[1] + lo[1]) * (T(3) * al) + (up[3] + lo[3]) * (T(3) * ar);
+        D = (up[0] - lo[0]) * (T(3) * bl) + (up[1] - lo[1]) * (al + bl) + (up[2] - lo[2]) * (T(3) * br) +
+            (up[3] - lo[3]) * (ar + br);
+    };
+    T lo[4], up[4], S, D, own, own_next, unused;
+    operand(Ra, lo, unused);
+    operand(Rb, up, own);
+    layer(kb - 1, Lb, lo, up, S, D);
+    T acc = S + D;
     double dot = 0.;
-    for (int P = P0; P < ke; ++P) {
-        const bool has_next = (P + 1) < n1;
-        T bot0 = T(0), bot1 = T(0), top0 = T(0), top1 = T(0);
-        T s_next = T(0), d_next = T(0);
-        if (has_next) {
-            load_row(P + 1, buf ^ 1, own_next, dir_next, FUSEP && (P + 1) < ke);
-            T a = T(0), b = T(0);
-            if (evalid) {
-                long long e = (long long)P * (n0 - 1) + tx;
-                T h = g.hy[P];
-                a = kh[e] * (gxf * h);
-                b = kv[e] * (gyf / h);
-            }
-            __syncthreads();
-            if (nvalid) {
-                T v0 = xs[(buf ^ 1) * PX + tx], v1 = xs[(buf ^ 1) * PX + tx + 1];
-                s_next = v0 + v1;
-                d_next = v1 - v0;
-                // w[x p][z q]: (s,s) eigenvalue 0, (d,s) 3a, (s,d) 3b, (d,d) a+b
-                T wds = (d_next + d_cur) * (T(3) * a);
-                T wsd = (s_next - s_cur) * (T(3) * b);
-                T wdd = (d_next - d_cur) * (a + b);
-                bot0 = -wsd;
-                top0 = wsd;
-                bot1 = wds - wdd;
-                top1 = wds + wdd;
+    Row cur = Rb;
+    for (int k0 = kb; k0 < ke; k0 += U) {
+        if (k0 > kb) {
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                load_row(k0 + 1 + u, R[u]);
+                load_layer(k0 + u, L[u]);
             }
         }
-        if (P >= kb) {
-            if (nvalid) {
-                T t0 = acc0 + bot0, t1 = acc1 + bot1;
-                oc[0 * PX + tx + 1] = t0 - t1;  // corner at node tx
-                oc[1 * PX + tx + 1] = t0 + t1;  // corner at node tx+1
-            }
-            __syncthreads();
-            if (nvalid) {
-                long long node = (long long)P * n0 + tx;
-                T s = oc[0 * PX + tx + 1] + oc[1 * PX + tx];
-                if (g.dsh) s += g.dsh[node] * own_cur;
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int k = k0 + u;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) lo[q] = up[q];
+            operand(R[u], up, own_next);
+            layer(k, L[u], lo, up, S, D);
+            if (k < ke) {
+                const long long node = (long long)k * n0 + i;
+                if (FUSEP) {
+                    pout[node] = own;
+                    xsol[node] = cur.x + alpha_prev * cur.p[1];
+                }
+                const T s = acc + (S - D) + cur.ds * own;
+                const bool fixed = cur.d[1] & 1u;
                 T out;
-                if (MODE == MODE_OP) out = dir_cur ? own_cur : s;
-                else out = dir_cur ? T(0) : (F[node] - s);
+                if (MODE == MODE_OP) out = fixed ? own : s;
+                else out = fixed ? T(0) : (cur.f - s);
                 y[node] = out;
-                if (DOT && !dir_cur) dot += (double)own_cur * (double)out;
+                if (DOT && !fixed) dot += (double)own * (double)out;
             }
+            acc = S + D;
+            own = own_next;
+            cur = R[u];
         }
-        acc0 = top0;
-        acc1 = top1;
-        s_cur = s_next;
-        d_cur = d_next;
-        own_cur = own_next;
-        dir_cur = dir_next;
-        buf ^= 1;
     }
     if (DOT) {
         double v[1] = {dot}, tot[1];
@@ -1500,29 +1522,47 @@ __host__ __device__ inline int part_lds_values(int P, int CB, int S) {
     return 6 * (S + (part_scan_width(P, CB, S) ? P : 0));
 }
 
-// The line factors of a thread's segment: a and w of every plane; c' only of the separator
-// (its coupling upwards), the interior ones are c'_u = a_(u+1) w_u (the coupling to the next
-// interior plane times the pivot inverse, as the set-up forms them), 0 on the last.
+// A vector's values of a thread's segment, 0 past its end.  No branch per value (each would wait
+// for the kernel arguments of its address anew): threads and planes past the end read the
+// segment's first plane, or node 0, and drop it.  Long segments skip the selects where a wave
+// holds whole ones (16 planes FP32, 96 x 96 x 192 nodes: 15.0 us with them, 12.6 without, 13.4
+// with branches; 4 planes FP64, 25 x 19 x 37 nodes: 4.3 us, with branches 4.6; 8 planes with the
+// residual update, 128 x 128 x 256: 42 us, with branches 47.6).
 template <typename T, int M>
-__device__ __forceinline__ void part_factors(const PartPos& q, long long plane, const T* __restrict__ la,
-                                             const T* __restrict__ lw, const T* __restrict__ lcp, T (&av)[M], T (&wv)[M],
-                                             T (&cv)[M]) {
-    T cs = T(0);
-    if (q.sep) cs = lcp[q.base + (long long)(q.len - 1) * plane];
+__device__ __forceinline__ void part_load(const PartPos& q, long long plane, const T* __restrict__ v, T (&out)[M]) {
+    if (M >= 16 && __all(q.len == M)) {  // a wave of whole segments
 #pragma unroll
-    for (int u = 0; u < M; ++u) {
-        av[u] = wv[u] = T(0);
-        if (u < q.len) {
-            const long long node = q.base + (long long)u * plane;
-            av[u] = la[node];
-            wv[u] = lw[node];
-        }
+        for (int u = 0; u < M; ++u) out[u] = v[q.base + (long long)u * plane];
+        return;
     }
+    const long long b = q.act ? q.base : 0;
+#pragma unroll
+    for (int u = 0; u < M; ++u) out[u] = v[b + (u < q.len ? (long long)u * plane : 0)];
+#pragma unroll
+    for (int u = 0; u < M; ++u) out[u] = u < q.len ? out[u] : T(0);
+}
+
+// The factors of a thread's segment: a and w of every plane; c' only of the separator (its
+// coupling upwards), the interior ones are c'_u = a_(u+1) w_u (the coupling to the next interior
+// plane times the pivot inverse, as the set-up forms them), 0 on the last; and the Thomas
+// factors a, w, c' of the separator's row of the column's separator system (0 without one).
+template <typename T, int M>
+__device__ __forceinline__ void part_factors(const PartPos& q, int P, int ncol, long long plane, const T* __restrict__ la,
+                                             const T* __restrict__ lw, const T* __restrict__ lcp,
+                                             const T* __restrict__ schur, T (&av)[M], T (&wv)[M], T (&cv)[M], T (&sv)[3]) {
+    const long long bs = q.sep ? q.base + (long long)(q.len - 1) * plane : 0;
+    const long long js = q.sep ? (long long)q.seg * ncol + q.col : 0, ss = q.sep ? (long long)(P - 1) * ncol : 0;
+    const T cl = lcp[bs], s0 = schur[js], s1 = schur[js + ss], s2 = schur[js + 2 * ss];
+    part_load<T, M>(q, plane, la, av);
+    part_load<T, M>(q, plane, lw, wv);
+    sv[0] = q.sep ? s0 : T(0);
+    sv[1] = q.sep ? s1 : T(0);
+    sv[2] = q.sep ? s2 : T(0);
 #pragma unroll
     for (int u = 0; u < M; ++u) {
         cv[u] = T(0);
         if (u + 1 < M) cv[u] = u + 1 < q.lint ? av[u + 1] * wv[u] : T(0);
-        if (q.sep && u == q.len - 1) cv[u] = cs;
+        if (q.sep && u == q.len - 1) cv[u] = cl;
     }
 }
 
@@ -1534,8 +1574,8 @@ __device__ __forceinline__ void part_factors(const PartPos& q, long long plane, 
 // (segment-major), with one pad per row where the scan runs, so that the lanes of a
 // column's scan, which step through the rows, fall in different banks.
 template <typename T, int M>
-__device__ inline void part_solve(const PartPos& q, int P, int CB, int ncol, const T* __restrict__ schur, T* lds,
-                                  const T (&rv)[M], const T (&av)[M], const T (&wv)[M], const T (&cv)[M], T (&zv)[M]) {
+__device__ inline void part_solve(const PartPos& q, int P, int CB, T* lds, const T (&rv)[M], const T (&av)[M],
+                                  const T (&wv)[M], const T (&cv)[M], const T (&sv)[3], T (&zv)[M]) {
     const int S = blockDim.x, W = part_scan_width(P, CB, S);
     const int CS = W ? CB + 1 : CB, SP = part_lds_values(P, CB, S) / 6;
     T* s_yf = lds;
@@ -1546,13 +1586,6 @@ __device__ inline void part_solve(const PartPos& q, int P, int CB, int ncol, con
     T* s_sc = s_sw + SP;
     const int t = q.t, cl = q.cl, seg = q.seg;
     const int pt = seg * CS + cl;  // the thread's slot (threads past CB * P have none)
-    // the separator factors (zero for the columns past the grid) travel while the interior is solved
-    T fa = T(0), fw = T(0), fc = T(0);
-    if (q.sep) {
-        fa = schur[(size_t)seg * ncol + q.col];
-        fw = schur[(size_t)(P - 1 + seg) * ncol + q.col];
-        fc = schur[(size_t)(2 * (P - 1) + seg) * ncol + q.col];
-    }
     // interior solve with the separators at zero
     T d[M];
     T dp = T(0);
@@ -1583,9 +1616,9 @@ __device__ inline void part_solve(const PartPos& q, int P, int CB, int ncol, con
             ehi = cv[u];
         }
     if (seg < P - 1) {
-        s_sa[pt] = fa;
-        s_sw[pt] = fw;
-        s_sc[pt] = fc;
+        s_sa[pt] = sv[0];
+        s_sw[pt] = sv[1];
+        s_sc[pt] = sv[2];
     }
     if (seg < P) {
         s_yf[pt] = q.act ? d[0] : T(0);
@@ -1706,19 +1739,14 @@ __global__ __launch_bounds__((PartLB<T, M>::value)) void k_cg_part(
     int ncol, int n, int P, int CB, long long plane, T* __restrict__ r, const T* __restrict__ q,
     const T* __restrict__ la, const T* __restrict__ lw, const T* __restrict__ lcp, const T* __restrict__ schur,
     T* __restrict__ z, PcgState* __restrict__ st, double* __restrict__ partials) {
-    if (!START && st->done) return;
     extern __shared__ __align__(16) unsigned char part_smem[];
     const PartPos pp = part_pos(ncol, n, P, CB, plane, M, (int)blockIdx.x);
-    T rv[M], av[M], wv[M], cv[M], qv[M];
-#pragma unroll
-    for (int u = 0; u < M; ++u) {
-        if (u < pp.len) {
-            const long long node = pp.base + (long long)u * plane;
-            rv[u] = r[node];
-            if (!START) qv[u] = q[node];
-        }
-    }
-    part_factors<T, M>(pp, plane, la, lw, lcp, av, wv, cv);
+    T rv[M], av[M], wv[M], cv[M], sv[3], qv[M];
+    part_load<T, M>(pp, plane, r, rv);
+    if (!START) part_load<T, M>(pp, plane, q, qv);
+    part_factors<T, M>(pp, P, ncol, plane, la, lw, lcp, schur, av, wv, cv, sv);
+    issue_loads();
+    if (!START && st->done) return;
     const T alpha = START ? T(0) : T(st->alpha);
     double rr = 0., rz = 0.;
 #pragma unroll
@@ -1732,7 +1760,7 @@ __global__ __launch_bounds__((PartLB<T, M>::value)) void k_cg_part(
         }
     }
     T zv[M];
-    part_solve<T, M>(pp, P, CB, ncol, schur, reinterpret_cast<T*>(part_smem), rv, av, wv, cv, zv);
+    part_solve<T, M>(pp, P, CB, reinterpret_cast<T*>(part_smem), rv, av, wv, cv, sv, zv);
 #pragma unroll
     for (int u = 0; u < M; ++u) {
         if (u < pp.len) {
@@ -1795,7 +1823,6 @@ __global__ __launch_bounds__((PartLB<T, M>::value)) void k_mg_smooth(
     T* xout, const T* __restrict__ rp, T omega, const T* __restrict__ la, const T* __restrict__ lw,
     const T* __restrict__ lcp, const T* __restrict__ schur, PcgState* __restrict__ st,
     double* __restrict__ partials, MgXfer<T> xf, int xcd) {
-    if (st->done) return;
     extern __shared__ __align__(16) unsigned char part_smem[];
     // XCD-aware order (xcd != 0, grid a multiple of 8): hardware block b runs on XCD b % 8;
     // each XCD takes a contiguous range of column groups, i.e. of the in-plane rows that
@@ -1804,8 +1831,7 @@ __global__ __launch_bounds__((PartLB<T, M>::value)) void k_mg_smooth(
     // still join the grid reduction.
     const int blk = xcd ? (int)(blockIdx.x & 7) * (int)(gridDim.x >> 3) + (int)(blockIdx.x >> 3) : (int)blockIdx.x;
     const PartPos pp = part_pos(ncol, n, P, CB, plane, M, blk);
-    T rv[M], av[M], wv[M], cv[M];
-    const T alpha = UPD ? T(st->alpha) : T(0);
+    T rv[M], qv[M], av[M], wv[M], cv[M], sv[3];
     // transfer tables of this thread's column (XF 1: its fine support; XF 2: its coarse cell)
     int ii[3] = {0, 0, 0}, jj[3] = {0, 0, 0};
     T wi[3] = {T(0), T(0), T(0)}, wj[3] = {T(0), T(0), T(0)};
@@ -1814,33 +1840,42 @@ __global__ __launch_bounds__((PartLB<T, M>::value)) void k_mg_smooth(
         mg_restrict_axis(ccol % xf.n0c, xf.n0c, xf.cx, xf.mx, xf.wx, ii, wi);
         mg_restrict_axis(ccol / xf.n0c, xf.n1c, xf.cy, xf.my, xf.wy, jj, wj);
     }
+    if constexpr (XF == 1) {
+        T src[M];
 #pragma unroll
-    for (int u = 0; u < M; ++u) {
-        if (u < pp.len) {
-            const long long node = pp.base + (long long)u * plane;
-            if constexpr (XF == 1) {
-                const long long k = (long long)pp.seg * M + u;
-                const T* src = xf.src + k * (long long)xf.n0f * xf.n1f;
-                T s = T(0);
+        for (int u = 0; u < M; ++u) {
+            const long long k = pp.act && u < pp.len ? (long long)pp.seg * M + u : 0;
+            const T* f = xf.src + k * (long long)xf.n0f * xf.n1f;
+            src[u] = T(0);
 #pragma unroll
-                for (int b = 0; b < 3; ++b) {
-                    const T* row = src + (long long)jj[b] * xf.n0f;
-                    s += wj[b] * (wi[0] * row[ii[0]] + wi[1] * row[ii[1]] + wi[2] * row[ii[2]]);
-                }
-                rv[u] = dbit(xf.dmask, node) ? T(0) : s;
-                r[node] = rv[u];
-            } else {
-                rv[u] = r[node];
-            }
-            if (UPD) {
-                rv[u] = rv[u] - alpha * q[node];
-                r[node] = rv[u];
+            for (int b = 0; b < 3; ++b) {
+                const T* row = f + (long long)jj[b] * xf.n0f;
+                src[u] += wj[b] * (wi[0] * row[ii[0]] + wi[1] * row[ii[1]] + wi[2] * row[ii[2]]);
             }
         }
+#pragma unroll
+        for (int u = 0; u < M; ++u) {
+            const bool fixed = u >= pp.len || dbit(xf.dmask, pp.base + (long long)u * plane);
+            rv[u] = fixed ? T(0) : src[u];
+        }
+    } else {
+        part_load<T, M>(pp, plane, r, rv);
     }
-    part_factors<T, M>(pp, plane, la, lw, lcp, av, wv, cv);
+    if (UPD) part_load<T, M>(pp, plane, q, qv);
+    part_factors<T, M>(pp, P, ncol, plane, la, lw, lcp, schur, av, wv, cv, sv);
+    issue_loads();
+    if (st->done) return;
+    if (UPD || XF == 1) {
+        const T alpha = UPD ? T(st->alpha) : T(0);
+#pragma unroll
+        for (int u = 0; u < M; ++u)
+            if (u < pp.len) {
+                if (UPD) rv[u] = rv[u] - alpha * qv[u];
+                r[pp.base + (long long)u * plane] = rv[u];
+            }
+    }
     T zv[M];
-    part_solve<T, M>(pp, P, CB, ncol, schur, reinterpret_cast<T*>(part_smem), rv, av, wv, cv, zv);
+    part_solve<T, M>(pp, P, CB, reinterpret_cast<T*>(part_smem), rv, av, wv, cv, sv, zv);
     double rz = 0., rr = 0.;
     MgProl<T> pr;
     if constexpr (XF == 2) {

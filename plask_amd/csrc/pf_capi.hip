@@ -82,6 +82,8 @@ struct pf_ctx {
     // geometry (FP64 and FP32 copies)
     double *hx = nullptr, *hy = nullptr, *hz = nullptr, *rmid = nullptr;
     float *hx32 = nullptr, *hy32 = nullptr, *hz32 = nullptr, *rmid32 = nullptr;
+    double* rhl = nullptr;  // 2D: 1 / element size along the layer axis
+    float* rhl32 = nullptr;
     // element data
     double *kh = nullptr, *kv = nullptr, *q = nullptr;
     float *kh32 = nullptr, *kv32 = nullptr;
@@ -581,10 +583,13 @@ static int tile_planes(int BY, int n1, int n2, int kmax) {
     return KC;
 }
 
-// 2D: rows of axis 1 per block, short enough for about one block per CU
-static int rows2d(int n1) {
-    int KC = 64;
-    while (KC > 1 && (n1 + KC - 1) / KC < 256) KC >>= 1;
+// 2D: rows of axis 1 per thread: long marches reuse the neighbouring rows, short ones give the
+// small grids enough waves (and keep n0 * chunks in 31 bits).  A multigrid solve of 200 x 400
+// nodes takes 1.97 ms with these (1 row on its coarse levels, 2 on the solve grid).
+static int rows2d(long long n0, long long n1) {
+    const long long N = n0 * n1;
+    int KC = N >= 4000000 ? 16 : N >= 1000000 ? 8 : N >= 240000 ? 4 : N >= 60000 ? 2 : 1;
+    while ((n1 + KC - 1) / KC * n0 >= (1LL << 30)) KC *= 2;
     return KC;
 }
 
@@ -630,6 +635,16 @@ int pf_grid_set(pf_ctx* ctx, int dim, int geom, const double* ax0, int64_t n0, c
         if ((rc = dalloc(ctx, hf[a], h.size()))) return rc;
         HIPCK(hipMemcpy(*hd[a], h.data(), sizeof(double) * h.size(), hipMemcpyHostToDevice));
         HIPCK(hipMemcpy(*hf[a], hf32.data(), sizeof(float) * h.size(), hipMemcpyHostToDevice));
+        if (dim == 2 && a == 1) {
+            for (size_t i = 0; i < h.size(); ++i) {
+                hf32[i] = 1.f / hf32[i];
+                h[i] = 1. / h[i];
+            }
+            if ((rc = dalloc(ctx, &ctx->rhl, h.size()))) return rc;
+            if ((rc = dalloc(ctx, &ctx->rhl32, h.size()))) return rc;
+            HIPCK(hipMemcpy(ctx->rhl, h.data(), sizeof(double) * h.size(), hipMemcpyHostToDevice));
+            HIPCK(hipMemcpy(ctx->rhl32, hf32.data(), sizeof(float) * h.size(), hipMemcpyHostToDevice));
+        }
     }
     if (geom == PF_GEOM_CYLINDRICAL) {
         std::vector<double> rm(n0 - 1);
@@ -712,7 +727,7 @@ int pf_grid_set(pf_ctx* ctx, int dim, int geom, const double* ax0, int64_t n0, c
         const int kind = tile_lds(by, (int)n0) > 65536 ? 1 : 0;
         ctx->apply_kind[0] = ctx->apply_kind[1] = kind;
     } else {
-        ctx->KC2 = rows2d((int)n1);
+        ctx->KC2 = rows2d(n0, n1);
     }
     ctx->upd_blocks = grid1(N, 256, 1024);
     size_t napply = 0;
@@ -725,7 +740,7 @@ int pf_grid_set(pf_ctx* ctx, int dim, int geom, const double* ax0, int64_t n0, c
         const size_t nrow = (size_t)n1 * ((n2 + 3) / 4) + 8;
         napply = std::max(napply, nrow);
     } else {
-        napply = (size_t)((n1 + ctx->KC2 - 1) / ctx->KC2);
+        napply = (size_t)(N + 255) / 256;  // k_apply2d with one row per thread
     }
     ctx->npartials = 2 * std::max<size_t>(napply, 4096);
     if ((rc = dalloc(ctx, &ctx->partials, ctx->npartials))) return rc;
@@ -902,10 +917,11 @@ template <> Axes3<float> axes3<float>(pf_ctx* ctx) {
 }
 template <typename T> static Axes2<T> axes2(pf_ctx* ctx);
 template <> Axes2<double> axes2<double>(pf_ctx* ctx) {
-    return Axes2<double>{(int)ctx->n[0], (int)ctx->n[1], ctx->hx, ctx->hy, ctx->rmid, ctx->dsh_on ? ctx->dsh : nullptr};
+    return Axes2<double>{(int)ctx->n[0], (int)ctx->n[1], ctx->hx, ctx->hy, ctx->rhl, ctx->rmid,
+                         ctx->dsh_on ? ctx->dsh : nullptr};
 }
 template <> Axes2<float> axes2<float>(pf_ctx* ctx) {
-    return Axes2<float>{(int)ctx->n[0], (int)ctx->n[1], ctx->hx32, ctx->hy32, ctx->rmid32,
+    return Axes2<float>{(int)ctx->n[0], (int)ctx->n[1], ctx->hx32, ctx->hy32, ctx->rhl32, ctx->rmid32,
                         ctx->dsh_on ? ctx->dsh32 : nullptr};
 }
 
@@ -922,6 +938,19 @@ template <typename T, int MODE> static void bnd_apply(pf_ctx* ctx, const T* x, T
 // residual forms include the boundary matrix; the fused CG forms do not (run_cg switches
 // to the unfused step when one is set) and neither does MODE_RESG (multigrid residuals:
 // the preconditioner sees the boundary matrix's diagonal only).
+template <typename T, int MODE, bool FUSEP, bool DOT>
+static void launch_apply2d(pf_ctx* ctx, const Axes2<T>& g, int KC, const T* xin, const T* zin, const T* pin, T* pout,
+                           T* y, const T* F, const uint64_t* dmask, const T* kh, const T* kv, T* xsol) {
+    const dim3 grid(((long long)((g.n1 + KC - 1) / KC) * g.n0 + 255) / 256);
+#define PF_APPLY2D(U)                                                                                                \
+    pf_launch(ctx, (k_apply2d<T, MODE, FUSEP, DOT, U>), grid, dim3(256), 0, ctx->stream, g, KC, xin, zin, pin, pout, \
+              xsol, y, F, dmask, kh, kv, ctx->st, ctx->partials)
+    if (KC == 1) PF_APPLY2D(1);
+    else if (KC == 2) PF_APPLY2D(2);
+    else PF_APPLY2D(4);
+#undef PF_APPLY2D
+}
+
 template <typename T, int MODE, bool FUSEP, bool DOT>
 static void launch_apply(pf_ctx* ctx, const T* xin, const T* zin, const T* pin, T* pout, T* y, const T* F, const T* kh,
                          const T* kv, T* xsol = nullptr, bool raw = false, MgProl<T> pr = MgProl<T>()) {
@@ -961,12 +990,8 @@ static void launch_apply(pf_ctx* ctx, const T* xin, const T* zin, const T* pin, 
                                g3, BY, KC, ytiles, nb, xo, xin, zin, pin, pout, xsol, y, F, dmask, kh, kv, ctx->st,
                                ctx->partials, pr);
     } else {
-        const int BX = (int)ctx->n[0];
-        int zt = (int)((ctx->n[1] + ctx->KC2 - 1) / ctx->KC2);
-        size_t shm = sizeof(T) * (size_t)(4 * (BX + 1));
         if constexpr (MODE != MODE_RESP)
-            pf_launch(ctx, (k_apply2d<T, MODE, FUSEP, DOT>), dim3(zt), dim3(BX), shm, ctx->stream, g2,
-                               ctx->KC2, xin, zin, pin, pout, xsol, y, F, dmask, kh, kv, ctx->st, ctx->partials);
+            launch_apply2d<T, MODE, FUSEP, DOT>(ctx, g2, ctx->KC2, xin, zin, pin, pout, y, F, dmask, kh, kv, xsol);
     }
     if constexpr (!FUSEP && !DOT && (MODE == MODE_OP || MODE == MODE_RES)) {
         if (ctx->have_bnd && !raw) bnd_apply<T, MODE>(ctx, xin, y, nullptr);
@@ -1294,7 +1319,7 @@ static int mg_refresh(pf_ctx* ctx) {
             hipLaunchKernelGGL(k_line_bc3d, dim3(gl), dim3(256), 0, ctx->stream, g, L.kh, L.kv, L.dmask, ctx->sb,
                                ctx->sc);
         } else {
-            const Axes2<double> g{L.n0, n2, L.hx, ctx->hy, L.rmid, ctx->dsh_on ? L.dsh : nullptr};
+            const Axes2<double> g{L.n0, n2, L.hx, ctx->hy, ctx->rhl, L.rmid, ctx->dsh_on ? L.dsh : nullptr};
             hipLaunchKernelGGL(k_line_bc2d, dim3(gl), dim3(256), 0, ctx->stream, g, L.kh, L.kv, L.dmask, ctx->sb,
                                ctx->sc);
         }
@@ -1458,6 +1483,7 @@ template <> struct MgPick<double> {
     static double* r0(const pf_ctx* c) { return c->mg_r0; }
     static const double* hy(const pf_ctx* c) { return c->hy; }
     static const double* hz(const pf_ctx* c) { return c->hz; }
+    static const double* rhl(const pf_ctx* c) { return c->rhl; }
     static const MgLevel& lv(const pf_ctx* c, int l) { return c->mg[l - 1]; }
     static int pm(const MgLevel& L) { return L.pm64; }
     static const double* hx(const MgLevel& L) { return L.hx; }
@@ -1489,6 +1515,7 @@ template <> struct MgPick<float> {
     static float* r0(const pf_ctx* c) { return c->mg_r0_32; }
     static const float* hy(const pf_ctx* c) { return c->hy32; }
     static const float* hz(const pf_ctx* c) { return c->hz32; }
+    static const float* rhl(const pf_ctx* c) { return c->rhl32; }
     static const MgLevel& lv(const pf_ctx* c, int l) { return c->mg[l - 1]; }
     static int pm(const MgLevel& L) { return L.pm32; }
     static const float* hx(const MgLevel& L) { return L.hx32; }
@@ -1538,7 +1565,7 @@ static MgView<T> mg_view(pf_ctx* ctx, int l, T* r0, T* z0) {
     v.pm = S::pm(L);
     const T* dl = ctx->dsh_on ? S::dsh(L) : nullptr;
     if (ctx->dim == 3) v.g = Axes3<T>{L.n0, L.n1, v.planes, S::hx(L), S::hyl(L), S::hz(ctx), dl};
-    else v.g2 = Axes2<T>{L.n0, v.planes, S::hx(L), S::hy(ctx), S::rmid(L), dl};
+    else v.g2 = Axes2<T>{L.n0, v.planes, S::hx(L), S::hy(ctx), S::rhl(ctx), S::rmid(L), dl};
     v.ncol = L.n0 * L.n1;
     v.kh = S::kh(L);
     v.kv = S::kv(L);
@@ -1569,14 +1596,8 @@ static void mg_residual_launch(pf_ctx* ctx, int l, const MgView<T>& v, MgProl<T>
         return;
     }
     if (ctx->dim == 2) {
-        // one block per chunk of KC rows of the layer axis, one thread per node of axis 0;
-        // short chunks on the (latency-bound) coarse levels
-        const int n0 = v.g2.n0, n1 = v.g2.n1;
-        const int KC = rows2d(n1);
-        pf_launch(ctx, (k_apply2d<T, MODE_RESG, false, false>), dim3((n1 + KC - 1) / KC), dim3(n0),
-                           sizeof(T) * 4 * (size_t)(n0 + 1), ctx->stream, v.g2, KC, (const T*)v.x, (const T*)nullptr,
-                           (const T*)nullptr, (T*)nullptr, (T*)nullptr, v.r, (const T*)v.b, v.dmask, v.kh, v.kv,
-                           ctx->st, ctx->partials);
+        launch_apply2d<T, MODE_RESG, false, false>(ctx, v.g2, rows2d(v.g2.n0, v.g2.n1), v.x, nullptr, nullptr, nullptr,
+                                                   v.r, v.b, v.dmask, v.kh, v.kv, nullptr);
         return;
     }
     const int n0 = v.g.n0, n1 = v.g.n1, n2 = v.g.n2;
@@ -1586,16 +1607,13 @@ static void mg_residual_launch(pf_ctx* ctx, int l, const MgView<T>& v, MgProl<T>
     const int nb = ytiles * ((n2 + KC - 1) / KC), grid = (nb + 7) / 8 * 8;
     const size_t shm = tile_lds(BY, n0) / sizeof(double) * sizeof(T);
     const int xo = ctx->mg_xcd ? 2 : ctx->xcd_order;
-    if (pr.xc)
-        pf_launch(ctx, (k_apply3d<T, MODE_RESP, false, false, 1>), dim3(grid), dim3(n0 * BY), shm, ctx->stream,
-                           v.g, BY, KC, ytiles, nb, xo, (const T*)v.x, (const T*)nullptr,
-                           (const T*)nullptr, (T*)nullptr, (T*)nullptr, v.r, (const T*)v.b, v.dmask, v.kh, v.kv,
-                           ctx->st, ctx->partials, pr);
-    else
-        pf_launch(ctx, (k_apply3d<T, MODE_RESG, false, false, 1>), dim3(grid), dim3(n0 * BY), shm, ctx->stream,
-                           v.g, BY, KC, ytiles, nb, xo, (const T*)v.x, (const T*)nullptr,
-                           (const T*)nullptr, (T*)nullptr, (T*)nullptr, v.r, (const T*)v.b, v.dmask, v.kh, v.kv,
-                           ctx->st, ctx->partials, pr);
+#define PF_MGRES(MODE)                                                                                              \
+    pf_launch(ctx, (k_apply3d<T, MODE, false, false, 1>), dim3(grid), dim3(n0 * BY), shm, ctx->stream, v.g, BY, KC, \
+              ytiles, nb, xo, (const T*)v.x, (const T*)nullptr, (const T*)nullptr, (T*)nullptr, (T*)nullptr, v.r,   \
+              (const T*)v.b, v.dmask, v.kh, v.kv, ctx->st, ctx->partials, pr)
+    if (pr.xc) PF_MGRES(MODE_RESP);
+    else PF_MGRES(MODE_RESG);
+#undef PF_MGRES
 }
 
 template <typename T>
@@ -3028,8 +3046,9 @@ int pf_set_launch(pf_ctx* ctx, int rows, int planes) {
         ctx->KC[0] = ctx->KC[1] = planes;
     } else {
         if (planes < 1) return fail(ctx, PF_EINVAL, "planes >= 1");
-        size_t need = 2 * (size_t)((ctx->n[1] + planes - 1) / planes);
-        if (need > ctx->npartials) return fail(ctx, PF_EINVAL, "too many blocks for the reduction buffer");
+        const int64_t chunks = (ctx->n[1] + planes - 1) / planes;
+        if (chunks > std::max<int64_t>(4096, (ctx->n[1] + 63) / 64) || chunks * ctx->n[0] >= (1LL << 30))
+            return fail(ctx, PF_EINVAL, "too many blocks for the reduction buffer");
         ctx->KC2 = planes;
     }
     drop_graphs(ctx);

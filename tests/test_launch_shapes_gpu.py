@@ -27,7 +27,8 @@ def _problem(shape, cyl=False):
 
 
 @pytest.mark.parametrize("shape", [(2, 2, 2), (17, 17, 5), (25, 19, 37), (128, 3, 9), (300, 2, 3), (65, 65, 8),
-                                   (2, 3), (33, 63), (33, 64), (33, 257), (700, 65)])
+                                   (2, 3), (33, 63), (33, 64), (33, 257), (700, 65), (300, 201), (600, 401),
+                                   (1000, 1001)])
 def test_default_launch_shapes_apply(shape):
     """y = A x (FP64) against the oracle's element sums: rounding of 27 products, 1e-13 of the largest."""
     g, axes, kh, kv, dn, c = _problem(shape)
@@ -38,6 +39,27 @@ def test_default_launch_shapes_apply(shape):
     ref = O.apply(g, 0, kh, kv, mask, x)
     y = c.apply(x)
     assert np.abs(y - ref).max() <= 1e-13 * np.abs(ref).max()
+    c.close()
+
+
+@pytest.mark.parametrize("rows", [1, 2, 3, 4, 7, 64])
+def test_rows_per_thread_2d(rows):
+    """The 2D operator with every unrolling and with remainders: plain (as above) and fused into
+    CG, whose solutions of one system (cond ~1e5, rtol 1e-12) agree to 1e-7 of their size."""
+    g, axes, kh, kv, dn, c = _problem((33, 65), cyl=True)
+    print("rows per thread", rows, flush=True)
+    mask = np.zeros(g.nnodes, np.uint8)
+    mask[dn] = 1
+    x = np.random.default_rng(1).uniform(-1, 1, g.nnodes)
+    c.set_source(np.random.default_rng(3).uniform(0, 1e16, g.nelems))
+    ref_t, _ = c.solve(x0=np.full(g.nnodes, 300.0), precision=PF_FP64, rtol=1e-12, precond=PRECOND_LINE)
+    c.set_launch(16, rows)
+    ref = O.apply(g, 0, kh, kv, mask, x)
+    assert np.abs(c.apply(x) - ref).max() <= 1e-13 * np.abs(ref).max()
+    for prec in (PF_FP64, PF_FP32_RELIABLE):
+        t, st = c.solve(x0=np.full(g.nnodes, 300.0), precision=prec, rtol=1e-12 if prec == PF_FP64 else 1e-10,
+                        precond=PRECOND_LINE)
+        assert st.status == 0 and np.abs(t - ref_t).max() <= 1e-7 * np.abs(ref_t).max()
     c.close()
 
 
