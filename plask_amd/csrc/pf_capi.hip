@@ -115,7 +115,7 @@ struct pf_ctx {
     float *x32 = nullptr, *r32 = nullptr, *p32 = nullptr, *q32 = nullptr, *z32 = nullptr, *dinv32 = nullptr;
     PcgState* st = nullptr;
     PcgState* hst = nullptr;  // pinned host mirror
-    double* partials = nullptr;
+    double *partials_mem = nullptr, *partials = nullptr;  // partials: behind the group tickets (last_block)
     size_t npartials = 0;
     bool dirty = true;  // F, Dinv, ||B|| need recomputing
     double bnorm = 0.;
@@ -574,12 +574,15 @@ static int tile_rows(int n0, int n1) {
     return best;
 }
 
-// Planes per block: kmax, halved until the grid has about 2 blocks per CU (aiming at 4 measured
-// slower: 65 x 65 columns 22.0 against 17.7 us per launch).
+// Planes per block: kmax, halved until the grid has 2 blocks per CU, or at 4 planes and less 1
+// (a block's first planes are read again by its neighbour, and every block costs the grid's
+// reduction a ticket).  Measured with 2 / 1 / this: 48 x 48 x 96 nodes, line preconditioner, 4.31 /
+// 3.88 / 3.79 ms; 96 x 96 x 192, FP32 preconditioner, 3.88 / 4.03 / 3.92 ms; 97 x 83 x 131 4.13 /
+// 4.11 / 4.11 ms.  Aiming at 4 measured slower (65 x 65 columns 22.0 against 17.7 us per launch).
 static int tile_planes(int BY, int n1, int n2, int kmax) {
     const long long ytiles = (n1 + BY - 2) / (BY - 1);
     int KC = kmax;
-    while (KC > 1 && (KC > n2 || ytiles * ((n2 + KC - 1) / KC) < 512)) KC >>= 1;
+    while (KC > 1 && (KC > n2 || ytiles * ((n2 + KC - 1) / KC) < (KC > 4 ? 512 : 256))) KC >>= 1;
     return KC;
 }
 
@@ -743,7 +746,10 @@ int pf_grid_set(pf_ctx* ctx, int dim, int geom, const double* ax0, int64_t n0, c
         napply = (size_t)(N + 255) / 256;  // k_apply2d with one row per thread
     }
     ctx->npartials = 2 * std::max<size_t>(napply, 4096);
-    if ((rc = dalloc(ctx, &ctx->partials, ctx->npartials))) return rc;
+    if ((rc = dalloc(ctx, &ctx->partials_mem, TICKET_DOUBLES + ctx->npartials))) return rc;
+    const std::vector<double> no_tickets(TICKET_DOUBLES, 0.);
+    HIPCK(hipMemcpy(ctx->partials_mem, no_tickets.data(), sizeof(double) * TICKET_DOUBLES, hipMemcpyHostToDevice));
+    ctx->partials = ctx->partials_mem + TICKET_DOUBLES;
     if ((rc = line_config(ctx))) return rc;
     ctx->dirty = true;
     return PF_OK;
@@ -1173,8 +1179,14 @@ static int prepare(pf_ctx* ctx) {
 }
 
 template <typename T, bool START>
-static void launch_part(pf_ctx* ctx, const PartShape& ps, int ncol, int n, long long plane, T* r, const T* q,
+static void launch_part(pf_ctx* ctx, PartShape ps, int ncol, int n, long long plane, T* r, const T* q,
                         const T* la, const T* lw, const T* lcp, const T* schur, T* z) {
+    // few columns: spread over at least 128 blocks (2304 columns of 96 planes: 72 blocks 4.92 ms
+    // per solve, 144 blocks 4.31, 288 blocks 4.54)
+    while (ps.CB > 8 && (ncol + ps.CB - 1) / ps.CB < 128) {
+        ps.CB >>= 1;
+        ps.threads = (ps.CB * part_threads(ps.P, 1024) + 63) / 64 * 64;
+    }
     const dim3 grid((ncol + ps.CB - 1) / ps.CB);
     const size_t lds = sizeof(T) * (size_t)part_lds_values(ps.P, ps.CB, ps.threads);
 #define PF_PART(MM)                                                                                            \
@@ -1657,8 +1669,9 @@ static void mg_smooth(pf_ctx* ctx, const MgView<T>& v, bool upd, int fin, T* r, 
     const int ncol = v.ncol, n = v.planes;
     PartShape ps = part_shape<T>(v.pm, n, ncol);
     // small coarse levels: fewer columns per block, so that the few columns spread over
-    // at least 64 blocks (larger levels keep full blocks, which measured faster)
-    while (ps.CB > 4 && (ncol + ps.CB - 1) / ps.CB < 64) {
+    // at least 128 blocks (larger levels keep full blocks, which measured faster; 64 blocks:
+    // 97 x 83 x 131 nodes 4.12 ms, 128: 4.08, 256: 4.23)
+    while (ps.CB > 4 && (ncol + ps.CB - 1) / ps.CB < 128) {
         ps.CB >>= 1;
         ps.threads = (ps.CB * part_threads(ps.P, 1024) + 63) / 64 * 64;
     }

@@ -63,6 +63,23 @@ def test_rows_per_thread_2d(rows):
     c.close()
 
 
+@pytest.mark.parametrize("rows,planes", [(2, 1), (3, 1), (4, 1), (4, 7), (31, 40)])
+def test_reductions_over_many_blocks(rows, planes):
+    """Grid reductions of one block, of 64 and less (one ticket) and of more (group tickets, the
+    last group short): every launch shape gives the same CG solve, cond ~1e5, rtol 1e-12."""
+    g, axes, kh, kv, dn, c = _problem((11, 30, 40))
+    c.set_source(np.random.default_rng(3).uniform(0, 1e16, g.nelems))
+    print("reductions", rows, planes, flush=True)
+    kw = dict(x0=np.full(g.nnodes, 300.0), precision=PF_FP64, rtol=1e-12)
+    ref, s0 = c.solve(precond=PRECOND_LINE, **kw)
+    c.set_launch(rows, planes)
+    for precond in (PRECOND_LINE, PRECOND_MG):
+        t, st = c.solve(precond=precond, **kw)
+        assert st.status == 0 and np.abs(t - ref).max() <= 1e-7 * np.abs(ref).max()
+        assert precond == PRECOND_MG or abs(st.iters - s0.iters) <= 2
+    c.close()
+
+
 @pytest.mark.parametrize("shape", [(3, 3, 192), (5, 4, 520), (4, 3, 521), (3, 4, 1024), (5, 520), (5, 521), (4, 1032),
                                    (4, 1033)])
 def test_long_lines_vcycle(shape):
