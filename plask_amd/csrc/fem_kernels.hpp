@@ -65,6 +65,7 @@ struct PcgState {
     double pap;      // (p, A p)
     double alpha;
     double rr;       // (r, r)
+    double rr0;      // (r, r) at the start of the run
     double stop2;    // stop when rr <= stop2
     double bb;       // (b, b)
     double beta0;    // beta of the first iteration: 0, or (r,z)/(r,z)_prev when a run resumes
@@ -932,7 +933,7 @@ __device__ inline void finish_start(PcgState* st, const double (&tot)[2]) {
     st->rz = tot[0];
     st->rz_prev = tot[0];
     st->beta0 = st->beta0 > 0. ? tot[0] / st->beta0 : 0.;
-    st->rr = tot[1];
+    st->rr = st->rr0 = tot[1];
     st->iters = 0;
     st->status = 0;
     st->done = (tot[1] <= st->stop2) ? 1 : 0;

@@ -146,6 +146,7 @@ struct pf_ctx {
     double mg_omega = 0.65;     // damping of the line-Jacobi smoother
     // cached graphs of one chunk of iterations
     hipGraphExec_t graph64 = nullptr, graph32 = nullptr;
+    hipGraphExec_t graph_end[2] = {nullptr, nullptr};  // the last 2 iterations (run_cg)
     int graph_chunk[2] = {0, 0}, graph_key[2] = {-1, -1};  // what graph64 / graph32 hold
     bool prec32 = false;  // FP64 PCG with the preconditioner applied in FP32 (PF_FP64_PREC32)
 
@@ -240,6 +241,10 @@ template <typename T> static int dalloc(pf_ctx* ctx, T** ptr, size_t count) {
 static void drop_graphs(pf_ctx* ctx) {
     if (ctx->graph64) hipGraphExecDestroy(ctx->graph64);
     if (ctx->graph32) hipGraphExecDestroy(ctx->graph32);
+    for (hipGraphExec_t& g : ctx->graph_end) {
+        if (g) hipGraphExecDestroy(g);
+        g = nullptr;
+    }
     ctx->graph64 = ctx->graph32 = nullptr;
     ctx->graph_key[0] = ctx->graph_key[1] = -1;
 }
@@ -1972,20 +1977,37 @@ static int run_cg(pf_ctx* ctx, int precond, T* x, T* r, T* p, T* p2, T* q, T* z,
         // preconditioner set-up; anything else is captured anew
         const int gi = sizeof(T) == 8 ? 0 : 1;
         const int key = precond + (p32 ? 16 : 0);
-        if (!*gcache || ctx->graph_chunk[gi] != chunk || ctx->graph_key[gi] != key) {
-            if (*gcache) hipGraphExecDestroy(*gcache);
-            *gcache = nullptr;
+        auto capture = [&](hipGraphExec_t* exec, int iters) -> int {
             hipGraph_t graph;
             HIPCK(hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
-            for (int c = 0; c < chunk; ++c) one_iter(c);
+            for (int c = 0; c < iters; ++c) one_iter(c);
             HIPCK(hipStreamEndCapture(ctx->stream, &graph));
-            HIPCK(hipGraphInstantiate(gcache, graph, nullptr, nullptr, 0));
+            HIPCK(hipGraphInstantiate(exec, graph, nullptr, nullptr, 0));
             hipGraphDestroy(graph);
+            return PF_OK;
+        };
+        hipGraphExec_t* gend = &ctx->graph_end[gi];
+        if (!*gcache || ctx->graph_chunk[gi] != chunk || ctx->graph_key[gi] != key) {
+            if (*gcache) hipGraphExecDestroy(*gcache);
+            if (*gend) hipGraphExecDestroy(*gend);
+            *gcache = *gend = nullptr;
+            if (int rc = capture(gcache, chunk)) return rc;
             ctx->graph_chunk[gi] = chunk;
             ctx->graph_key[gi] = key;
         }
-        for (;;) {
-            HIPCK(hipGraphLaunch(*gcache, ctx->stream));
+        // Multigrid iterations past the stop are ~30 launches each that only find the flag (2.3 us
+        // each): where the mean reduction per iteration so far says that 2 iterations reach the
+        // stop, a graph of 2 runs instead of the chunk of 4 (25 x 19 x 37 nodes, 13 iterations;
+        // two replays of such a graph in place of the chunk cost 10 us more per chunk).
+        auto near_end = [&]() {
+            const PcgState& s = *ctx->hst;
+            const double per_iter = s.iters > 0 ? std::log(s.rr0 / s.rr) / s.iters : 0.;
+            return mg && chunk == 4 && per_iter > 0. && std::log(s.rr / s.stop2) <= 2. * per_iter;
+        };
+        for (bool end = false;; end = near_end()) {
+            if (end && !*gend)
+                if (int rc = capture(gend, 2)) return rc;
+            HIPCK(hipGraphLaunch(end ? *gend : *gcache, ctx->stream));
             HIPCK(hipMemcpyAsync(ctx->hst, ctx->st, sizeof(PcgState), hipMemcpyDeviceToHost, ctx->stream));
             HIPCK(hipStreamSynchronize(ctx->stream));
             if (ctx->hst->done) break;

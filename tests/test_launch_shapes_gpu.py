@@ -99,3 +99,19 @@ def test_long_lines_vcycle(shape):
     c.set_line_segment(0)
     assert np.abs(c.precond_apply(r, PF_FP64, PRECOND_LINE) - zl).max() <= 1e-10 * np.abs(zl).max()
     c.close()
+
+
+@pytest.mark.parametrize("rtol", [1e-3, 1e-6, 1e-8, 1e-10, 1e-12])
+def test_last_iterations_in_a_short_graph(rtol):
+    """The stop is met at another iteration of the chunk for every rtol; whether the last ones run
+    in the chunk's graph or in the short one, iterations and bits are those of checks every 2."""
+    g, axes, kh, kv, dn, c = _problem((17, 15, 24))
+    c.set_source(np.random.default_rng(3).uniform(0, 1e16, g.nelems))
+    print("short graph", rtol, flush=True)
+    kw = dict(x0=np.full(g.nnodes, 300.0), precision=PF_FP64, precond=PRECOND_MG)
+    for _ in range(3):  # replayed, and with another tolerance between
+        a, sa = c.solve(rtol=rtol, **kw)
+        c.solve(rtol=1e-5, **kw)
+    b, sb = c.solve(rtol=rtol, check_every=2, **kw)
+    assert sa.iters == sb.iters and np.array_equal(a, b)
+    c.close()
