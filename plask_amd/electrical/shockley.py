@@ -132,24 +132,26 @@ class _ShockleyBase(_sb.FemSolver):
             h = float(z[kt] - z[kb])
             heights.append(h)
             self._junctions.append((kb, kt, h))
-            for w in where:
-                if self.DIM == 2:
-                    k, i = int(w[0]), int(w[1])
-                    e = i + m[0] * k
-                    cols = [i, i + 1]
-                else:
-                    k, j, i = int(w[0]), int(w[1]), int(w[2])
-                    e = i + m[0] * (j + m[1] * k)
-                    cols = [i + n0 * j, i + 1 + n0 * j, i + n0 * (j + 1), i + 1 + n0 * (j + 1)]
-                elems.append(e)
-                bot.extend([cc + kb * plane for cc in cols])
-                top.extend([cc + kt * plane for cc in cols])
-                jid.append(n - 1)
-        self._jelems = np.array(elems, dtype=np.int64)
-        self._jid = np.array(jid, dtype=np.int32)
+            if self.DIM == 2:
+                k, i = where.T
+                elems.append(i + m[0] * k)
+                cols = np.stack([i, i + 1], axis=1)
+            else:
+                k, j, i = where.T
+                elems.append(i + m[0] * (j + m[1] * k))
+                cols = np.stack([i + n0 * j, i + 1 + n0 * j, i + n0 * (j + 1), i + 1 + n0 * (j + 1)], axis=1)
+            bot.append((cols + kb * plane).ravel())
+            top.append((cols + kt * plane).ravel())
+            jid.append(np.full(len(where), n - 1))
+
+        def joined(parts, dtype):
+            return np.concatenate(parts).astype(dtype) if parts else np.zeros(0, dtype)
+
+        self._jelems = joined(elems, np.int64)
+        self._jid = joined(jid, np.int32)
         c.set_start_cond(float(self._start_cond[1]), float(self._start_cond[0]))
-        c.set_junctions(self._jelems, 2 if self.DIM == 2 else 4, np.array(bot, dtype=np.int64),
-                        np.array(top, dtype=np.int64), list(self._jid), heights)
+        c.set_junctions(self._jelems, 2 if self.DIM == 2 else 4, joined(bot, np.int64), joined(top, np.int64),
+                        list(self._jid), heights)
         leaves = self._geometry._leaves
         air_noheat = True
         leaf_noheat = np.array([(lf[0].material is None or getattr(lf[0].material, "kind", "") == "empty" or
