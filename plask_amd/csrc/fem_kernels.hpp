@@ -1369,28 +1369,45 @@ __global__ void k_part_factor(int ncol, int n, int m, long long plane, const dou
         part_factor_segment<T>((int)(t % ncol), (int)(t / ncol), ncol, n, m, plane, bb, cc, la, lw, lcp, sff, sfl);
 }
 
-// LU recurrence of a column's separator system
+// LU recurrence of a column's separator system, one thread.  The operands of 8 separators are
+// read together, ahead of their steps of the recurrence: a memory latency for 8 separators
+// instead of one each.
 template <typename T>
 __device__ inline void part_schur_column(int col, int ncol, int n, int m, long long plane, const T* __restrict__ la,
                                          const T* __restrict__ lw, const T* __restrict__ lcp,
                                          const double* __restrict__ sff, const double* __restrict__ sfl,
                                          T* __restrict__ schur) {
-    const int P = (n + m - 1) / m;
+    constexpr int U = 8;
+    const int ns = (n + m - 1) / m - 1;
     double off_prev = 0., sc_prev = 0.;
-    for (int j = 0; j < P - 1; ++j) {
-        const long long ns = (long long)((j + 1) * m - 1) * plane + col;
-        const double elo = la[ns], bs = lw[ns], ehi = lcp[ns];
-        const double wl = lw[ns - plane];
-        const double ff = sff[(size_t)(j + 1) * ncol + col], fl = sfl[(size_t)(j + 1) * ncol + col];
-        const double sjj = bs - elo * elo * wl - ehi * ehi * ff;
-        const double soff = j + 1 < P - 1 ? -ehi * fl * (double)la[(long long)((j + 2) * m - 1) * plane + col] : 0.;
-        const double w = 1. / (sjj - off_prev * sc_prev);
-        const double cp = soff * w;
-        schur[(size_t)j * ncol + col] = T(off_prev);
-        schur[(size_t)(P - 1 + j) * ncol + col] = T(w);
-        schur[(size_t)(2 * (P - 1) + j) * ncol + col] = T(cp);
-        off_prev = soff;
-        sc_prev = cp;
+    for (int j0 = 0; j0 < ns; j0 += U) {
+        double elo[U], bs[U], ehi[U], wl[U], ff[U], fl[U], up[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int j = min(j0 + u, ns - 1), jn = min(j + 1, ns - 1);
+            const long long sep = (long long)((j + 1) * m - 1) * plane + col;
+            elo[u] = la[sep];
+            bs[u] = lw[sep];
+            ehi[u] = lcp[sep];
+            wl[u] = lw[sep - plane];
+            ff[u] = sff[(size_t)(j + 1) * ncol + col];
+            fl[u] = sfl[(size_t)(j + 1) * ncol + col];
+            up[u] = la[(long long)((jn + 1) * m - 1) * plane + col];
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int j = j0 + u;
+            if (j >= ns) break;
+            const double sjj = bs[u] - elo[u] * elo[u] * wl[u] - ehi[u] * ehi[u] * ff[u];
+            const double soff = j + 1 < ns ? -ehi[u] * fl[u] * up[u] : 0.;
+            const double w = 1. / (sjj - off_prev * sc_prev);
+            const double cp = soff * w;
+            schur[(size_t)j * ncol + col] = T(off_prev);
+            schur[(size_t)(ns + j) * ncol + col] = T(w);
+            schur[(size_t)(2 * ns + j) * ncol + col] = T(cp);
+            off_prev = soff;
+            sc_prev = cp;
+        }
     }
 }
 

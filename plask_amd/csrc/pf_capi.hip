@@ -1292,7 +1292,7 @@ static int mg_refresh(pf_ctx* ctx) {
                            L.kh, L.kh32);
         hipLaunchKernelGGL((k_convert<float, double>), dim3(grid1(L.E, 256, 4096)), dim3(256), 0, ctx->stream, L.E,
                            L.kv, L.kv32);
-        hipLaunchKernelGGL(k_mg_coarsen_mask, dim3(grid1((L.N + 63) / 64, 256, 4096)), dim3(256), 0, ctx->stream, tr,
+        hipLaunchKernelGGL(k_mg_coarsen_mask, dim3(grid1(L.N, 256, 4096)), dim3(256), 0, ctx->stream, tr,
                            F ? F->dmask : ctx->dmask, L.dmask);
         const int ncol = L.n0 * L.n1;
         // Segment lengths: with the default lengths (8 planes FP64, 16 FP32 on the solve
