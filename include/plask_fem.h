@@ -281,8 +281,8 @@ int pf_set_multigrid(pf_ctx* ctx, int max_levels, int coarse_sweeps, double omeg
 
 /* 3D multigrid: run the grid transfers inside the neighbouring kernels (restriction in a
  * coarse level's first sweep, prolongation in the residual and sweep that follow it; on = 1)
- * or as kernels of their own (0, the default: measured faster).  Same preconditioner
- * either way.  No reference counterpart (tuning hook). */
+ * or as kernels of their own (0, the default: measured faster) except for the restriction to
+ * the small FP64 levels.  Same preconditioner either way.  No reference counterpart (tuning hook). */
 int pf_set_multigrid_fusion(pf_ctx* ctx, int on);
 
 /* 3D multigrid, levels below the solve grid: residual tiles ordered by in-plane row and

@@ -1822,8 +1822,10 @@ __global__ __launch_bounds__((PartLB<T, M>::value)) void k_cg_part(
 // level the sweep works on; the tables are those between the two levels (mg_kernels.hpp).
 template <typename T> struct MgXfer {
     int n0f = 0, n1f = 0, n0c = 0, n1c = 0;
-    const int* cx = nullptr;
-    const int* cy = nullptr;
+    const int* rx = nullptr;  // restriction rows (MgTransfer) and their weights
+    const int* ry = nullptr;
+    const T* rwx = nullptr;
+    const T* rwy = nullptr;
     const int* mx = nullptr;
     const int* my = nullptr;
     const T* wx = nullptr;
@@ -1831,25 +1833,6 @@ template <typename T> struct MgXfer {
     const T* src = nullptr;
     const uint64_t* dmask = nullptr;
 };
-
-// the (up to) 3 fine nodes of coarse node I along one axis and their restriction
-// weights (absent ones repeat the first index with weight 0)
-template <typename T>
-__device__ __forceinline__ void mg_restrict_axis(int I, int nc, const int* __restrict__ cidx,
-                                                 const int* __restrict__ m, const T* __restrict__ w, int (&idx)[3],
-                                                 T (&wt)[3]) {
-    const int lo = I > 0 ? cidx[I - 1] + 1 : 0;
-    const int hi = I < nc - 1 ? cidx[I + 1] - 1 : cidx[I];
-#pragma unroll
-    for (int a = 0; a < 3; ++a) {
-        const int i = lo + a;
-        const bool ok = i <= hi;
-        idx[a] = ok ? i : lo;
-        const int mm = m[idx[a]];
-        const T ww = w[idx[a]];
-        wt[a] = ok ? (mm == I ? T(1) - ww : (mm + 1 == I ? ww : T(0))) : T(0);
-    }
-}
 
 // Damped line-Jacobi sweep of the multigrid smoother, same partitioned line solve:
 // xout = xin + omega T^-1 r (xin null: start from zero; xin may be xout).
@@ -1877,8 +1860,14 @@ __global__ __launch_bounds__((PartLB<T, M>::value)) void k_mg_smooth(
     T wi[3] = {T(0), T(0), T(0)}, wj[3] = {T(0), T(0), T(0)};
     const int ccol = pp.act ? pp.col : 0;
     if constexpr (XF == 1) {
-        mg_restrict_axis(ccol % xf.n0c, xf.n0c, xf.cx, xf.mx, xf.wx, ii, wi);
-        mg_restrict_axis(ccol / xf.n0c, xf.n1c, xf.cy, xf.my, xf.wy, jj, wj);
+        const int J = ccol / xf.n0c, I = ccol - J * xf.n0c;
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            ii[a] = xf.rx[3 * I + a];
+            wi[a] = xf.rwx[3 * I + a];
+            jj[a] = xf.ry[3 * J + a];
+            wj[a] = xf.rwy[3 * J + a];
+        }
     }
     if constexpr (XF == 1) {
         T src[M];

@@ -142,7 +142,7 @@ struct pf_ctx {
     int mg_max_levels = 0;      // 0: coarsen until both in-plane axes have <= 3 nodes
     int mg_coarse_sweeps = 1;   // smoothing sweeps on the coarsest level
     int mg_xcd = 1;             // multigrid levels >= 1: XCD-aligned residual tiles and sweep groups
-    int mg_fuse = 0;            // 3D: grid transfers fused into the smoother / residual kernels (measured slower)
+    int mg_fuse = 0;            // 3D: all grid transfers fused into the smoother / residual kernels (measured slower)
     double mg_omega = 0.65;     // damping of the line-Jacobi smoother
     // cached graphs of one chunk of iterations
     hipGraphExec_t graph64 = nullptr, graph32 = nullptr;
@@ -1708,8 +1708,10 @@ static MgXfer<T> mg_xfer(pf_ctx* ctx, int t, const MgView<T>& coarse, const T* s
     x.n1f = tr.n1f;
     x.n0c = tr.n0c;
     x.n1c = tr.n1c;
-    x.cx = tr.cx;
-    x.cy = tr.cy;
+    x.rx = tr.rx;
+    x.ry = tr.ry;
+    x.rwx = coarse.rwx;
+    x.rwy = coarse.rwy;
     x.mx = tr.mx;
     x.my = tr.my;
     x.wx = coarse.wx;
@@ -1740,6 +1742,13 @@ template <typename T>
 static void mg_vcycle(pf_ctx* ctx, T* r, const T* q, T* z, bool upd, int fin) {
     const int L = (int)ctx->mg.size() + 1;
     const bool fuse = ctx->mg_fuse && ctx->dim == 3 && L > 1 && ctx->apply_kind[sizeof(T) == 8 ? 0 : 1] == 0;
+    // restriction inside the level's first sweep: everywhere with fused transfers, and otherwise
+    // in FP64 on the 3D levels of 4-plane segments (at most 512 columns), where a launch costs more
+    // than the sweep's gather (2.7 us against 0.4 per level: 25 x 19 x 37 nodes 1.76 -> 1.70 ms,
+    // 97 x 83 x 131 3.93 -> 3.90; FP32, 96 x 96 x 192: 3.88 -> 3.91, so not there)
+    auto restricts = [&](const MgView<T>& v) {
+        return fuse || (sizeof(T) == 8 && ctx->dim == 3 && part_shape<T>(v.pm, v.planes, v.ncol).m == 4);
+    };
     // profiled chunks: level-0 kernels by kind, all coarse-level work as one record
     auto cat = [](int l, int kind) { return l == 0 ? kind : -1; };
     auto open = [&](int c) { return c >= 0 ? prof_open(ctx, c) : -1; };
@@ -1757,7 +1766,7 @@ static void mg_vcycle(pf_ctx* ctx, T* r, const T* q, T* z, bool upd, int fin) {
                 prof_close(ctx, h);
             }
             const int h = open(cat(l, PF_KCAT_MG_SMOOTH));
-            if (s == 0 && fuse && l > 0) {
+            if (s == 0 && l > 0 && restricts(v)) {
                 // b = R r of the finer level, read and stored by the sweep itself
                 const MgView<T> fv = mg_view<T>(ctx, l - 1, r, z);
                 const MgXfer<T> xf = mg_xfer<T>(ctx, l - 1, v, fv.r, v.dmask);
@@ -1774,8 +1783,8 @@ static void mg_vcycle(pf_ctx* ctx, T* r, const T* q, T* z, bool upd, int fin) {
             int h = open(cat(l, PF_KCAT_MG_RESIDUAL));
             mg_residual<T>(ctx, l, v);
             prof_close(ctx, h);
-            if (!fuse) {
-                const MgView<T> c = mg_view<T>(ctx, l + 1, r, z);
+            const MgView<T> c = mg_view<T>(ctx, l + 1, r, z);
+            if (!restricts(c)) {
                 const MgTransfer tr = mg_transfer(ctx, (size_t)l);
                 h = open(cat(l, PF_KCAT_MG_TRANSFER));
                 const int hk = prof_kern<T>(ctx, PF_K_RESTRICT, l,
