@@ -379,9 +379,8 @@ def config1(steps, with_cpu):
 
 def config3(cpu_seconds):
     """256 uneven 2D cylindrical Shockley instances (plask_amd.workloads.shockley_cyl_batch,
-    seeds 3000+i; 50x100 to 400x800 nodes): one persistent batched launch per solve
-    (multigrid-preconditioned CG inside each workgroup, Picard loop <= 30 on the device),
-    autotuned workgroup size / count.  CPU reference path (assembly + band Cholesky per
+    seeds 3000+i; 50x100 to 400x800 nodes): all instances advancing together, one
+    launch per step (multigrid-preconditioned CG, Picard loop <= 30 on the device).  CPU reference path (assembly + band Cholesky per
     Picard loop, serial oracle) on a bounded sample: one loop timed on a few instances, a
     cost model t = c N kd^2 (band Cholesky, kd = n_r + 1) fitted to them and summed over
     the loops every instance ran on the GPU."""
@@ -423,19 +422,17 @@ def config3(cpu_seconds):
     c = sum(dt for _, dt in cpu) / sum(work(i) for i, _ in cpu)
     cpu_total = c * sum(loops[i] * work(i) for i in range(len(insts)))
     # algorithmic bytes (FP64, each value read or written once per pass): per CG iteration
-    # the marched operator apply (p, two conductivities, q: 32 B/node), the x / r update
-    # (48), p = z + beta p and (r, z) (40) and the V-cycle, 232 B per node of every level
-    # (two line sweeps 56 + 64, two marched residuals 2 x 40, restriction 12, prolongation
-    # 20) over levels of 2 N nodes in all (axis 0 halved per level); per Picard loop the line
-    # factors and coarse conductivities of all levels, the junction update and the currents
-    # (~150 B/node)
+    # the apply with the direction and solution updates (64 B/node) and the V-cycle, 168 B per
+    # node of every level (first sweep 56, residual 40, way up 72) over levels of 2 N nodes in
+    # all (axis 0 halved per level); per Picard loop the line factors and coarse
+    # conductivities of all levels, the junction update and the currents (~150 B/node)
     nodes = (nr * nz).astype(np.float64)
-    bytes_alg = float(np.sum(nodes * (its * (32 + 48 + 40 + 232 * 2) + loops * 150)))
-    roofline = {"bound": "hbm", "kernel": "k_batch_shockley2d (whole batch)", "achieved": round(bytes_alg / t / 1e9, 1),
+    bytes_alg = float(np.sum(nodes * (its * (64 + 168 * 2) + loops * 150)))
+    roofline = {"bound": "hbm", "kernel": "k_bs_* (whole batch)", "achieved": round(bytes_alg / t / 1e9, 1),
                 "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(bytes_alg / t / 1e9 / HBM_PEAK_GBS, 4),
                 "traffic": None, "bytes": bytes_alg,
-                "note": "one workgroup per instance: each instance's passes are chains of dependent loads on one CU; "
-                        "the time is the slowest instances' (largest, most CG iterations), not the total bytes"}
+                "note": "late loops hold only the instances that have not converged: their steps are launches of few "
+                        "blocks, held by latency"}
     return dict(workload="shockley_cyl_batch_256", instances=len(insts), nodes_total=int((nr * nz).sum()),
                 roofline=roofline,
                 gpu_s=t, block=blk, workgroups=nwg, autotune_s=t_tune, picard_loops_mean=float(loops.mean()),

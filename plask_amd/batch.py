@@ -50,7 +50,7 @@ def _p(a):
 
 
 class ShockleyBatch:
-    """Many 2D Shockley problems solved by one persistent kernel launch."""
+    """Many 2D Shockley problems solved together on one GPU."""
 
     def __init__(self, instances, cylindrical=True, device=0):
         self.L = load_library()
@@ -94,8 +94,8 @@ class ShockleyBatch:
     def opts(self, maxloops=30, maxit=100000, maxerr=0.05, rtol=1e-8, stable=False, block=0, nwg=0, precond=3,
              loop_budget=5, progress=False):
         """precond 3: multigrid V-cycle per instance (the default), 2: line preconditioner.
-        loop_budget: Picard loops per kernel launch and instance (0: one launch for all);
-        progress: print a line after every launch."""
+        loop_budget: Picard loops between two progress reports (0: one report, at the end);
+        progress: print a line at every report."""
         return BatchOpts(maxloops, maxit, maxerr, rtol, 1 if stable else 0, block, nwg, int(precond),
                          int(loop_budget), _PRINT_PROGRESS if progress else _NO_PROGRESS, None)
 
