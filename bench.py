@@ -71,13 +71,13 @@ def kernel_bytes(shape, m=8):
     """Algorithmic HBM bytes per launch (FP64) of the kernels of one PCG iteration.
     apply_fused: read z, p_old, x; write p_new, q, x (48 B/node); k_xy, k_z
       (16 B/element); Dirichlet bitmask (N/8 B).
-    line (partitioned, segments of m planes): read r, q, a, w, c'; write r, z
-      (56 B/node); separator factors 3 x 8 B per separator per column.
+    line (partitioned, segments of m planes): read r, q, a, w; write r, z (48 B/node);
+      separator factors 4 x 8 B per separator per column.
     apply_plain: read x, write y (16 B/node), 16 B/element, bitmask.
     mg_residual (V-cycle, solve grid): r = b - A x: read x, b; write r (24 B/node),
       16 B/element, bitmask.
-    mg_smooth (V-cycle, solve grid): damped line sweep, first (read r, q, a, w, c';
-      write r, x) or last (read r_s, x, r, a, w, c'; write x): 56 B/node + separators.
+    mg_smooth (V-cycle, solve grid): damped line sweep, first (read r, q, a, w;
+      write r, x) or last (read r_s, x, r, a, w; write x): 48 B/node + separators.
     mg_transfer: restriction (read fine r, write coarse b) and prolongation (read coarse x,
       read and write fine x), averaged: 12 B per fine node + 8 B per coarse node.
     FP32 forms: half the bytes of vectors and element data (line: 16-plane segments)."""
@@ -88,12 +88,12 @@ def kernel_bytes(shape, m=8):
     P32 = (nz + 15) // 16
     Nc = (nx // 2 + 1 if nx > 3 else nx) * (ny // 2 + 1 if ny > 3 else ny) * nz
     return {"apply_fused": 48 * N + 16 * E + mask,
-            "line": 56 * N + 24 * (P - 1) * nx * ny,
+            "line": 48 * N + 32 * (P - 1) * nx * ny,
             "apply_plain": 16 * N + 16 * E + mask,
             "apply_fused_fp32": 24 * N + 8 * E + mask,
-            "line_fp32": 28 * N + 12 * (P32 - 1) * nx * ny,
+            "line_fp32": 24 * N + 16 * (P32 - 1) * nx * ny,
             "mg_residual": 24 * N + 16 * E + mask,
-            "mg_smooth": 56 * N + 24 * (P - 1) * nx * ny,
+            "mg_smooth": 48 * N + 32 * (P - 1) * nx * ny,
             "mg_transfer": 12 * N + 8 * Nc}
 
 
