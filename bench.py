@@ -80,7 +80,8 @@ def kernel_bytes(shape, m=8):
       write r, x) or last (read r_s, x, r, a, w; write x): 48 B/node + separators.
     mg_transfer: restriction (read fine r, write coarse b) and prolongation (read coarse x,
       read and write fine x), averaged: 12 B per fine node + 8 B per coarse node.
-    FP32 forms: half the bytes of vectors and element data (line: 16-plane segments)."""
+    FP32 forms: half the bytes of vectors and element data; line: 16-plane segments, reads
+      r, q, a, w, c' and writes r, z (28 B/node), separator factors 3 x 4 B."""
     nx, ny, nz = shape
     N, E = nx * ny * nz, (nx - 1) * (ny - 1) * (nz - 1)
     mask = 8 * ((N + 63) // 64)
@@ -91,7 +92,7 @@ def kernel_bytes(shape, m=8):
             "line": 48 * N + 32 * (P - 1) * nx * ny,
             "apply_plain": 16 * N + 16 * E + mask,
             "apply_fused_fp32": 24 * N + 8 * E + mask,
-            "line_fp32": 24 * N + 16 * (P32 - 1) * nx * ny,
+            "line_fp32": 28 * N + 12 * (P32 - 1) * nx * ny,
             "mg_residual": 24 * N + 16 * E + mask,
             "mg_smooth": 48 * N + 32 * (P - 1) * nx * ny,
             "mg_transfer": 12 * N + 8 * Nc}

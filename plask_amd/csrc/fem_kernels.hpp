@@ -1582,22 +1582,28 @@ __device__ __forceinline__ void part_load(const PartPos& q, long long plane, con
     for (int u = 0; u < M; ++u) out[u] = u < q.len ? out[u] : T(0);
 }
 
-// The factors of a thread's segment: a and w of every plane; c' only of the separator (its
-// coupling upwards), the interior ones are c'_u = a_(u+1) w_u (the coupling to the next interior
-// plane times the pivot inverse, as the set-up forms them), 0 on the last; and the Thomas
-// factors a, w, c' of the separator's row of the column's separator system (0 without one).
+// The factors of a thread's segment: a, w and c' of every plane, and the Thomas factors a, w, c'
+// of the separator's row of the column's separator system (0 without one).  FP64 reads c' only of
+// the separator (its coupling upwards): the interior ones are c'_u = a_(u+1) w_u (the coupling to
+// the next interior plane times the pivot inverse, the set-up's own product), 0 on the last.  FP32
+// reads them all: the set-up rounds the FP64 product once, the product of the two rounded factors
+// would be off by up to three (PF_FP64_PREC32 solve of 96 x 96 x 192 nodes: 4.27 ms, with the
+// product 4.20).
 template <typename T, int M>
 __device__ __forceinline__ void part_factors(const PartPos& q, int P, int ncol, long long plane, const T* __restrict__ la,
                                              const T* __restrict__ lw, const T* __restrict__ lcp,
                                              const T* __restrict__ schur, T (&av)[M], T (&wv)[M], T (&cv)[M], T (&sv)[3]) {
+    constexpr bool all = sizeof(T) == 4;
     const long long bs = q.sep ? q.base + (long long)(q.len - 1) * plane : 0;
     const long long js = q.sep ? (long long)q.seg * ncol + q.col : 0, ss = q.sep ? (long long)(P - 1) * ncol : 0;
-    const T cl = lcp[bs], s0 = schur[js], s1 = schur[js + ss], s2 = schur[js + 2 * ss];
+    const T cl = all ? T(0) : lcp[bs], s0 = schur[js], s1 = schur[js + ss], s2 = schur[js + 2 * ss];
     part_load<T, M>(q, plane, la, av);
     part_load<T, M>(q, plane, lw, wv);
+    if (all) part_load<T, M>(q, plane, lcp, cv);
     sv[0] = q.sep ? s0 : T(0);
     sv[1] = q.sep ? s1 : T(0);
     sv[2] = q.sep ? s2 : T(0);
+    if (all) return;
 #pragma unroll
     for (int u = 0; u < M; ++u) {
         cv[u] = T(0);

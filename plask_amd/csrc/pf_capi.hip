@@ -300,13 +300,18 @@ static double mask_bytes(long long n) { return 8.0 * (double)((n + 63) / 64); }
 static double bytes_apply_fused(long long n, long long e, int t) { return t * (6.0 * n + 2.0 * e) + mask_bytes(n); }
 // residual r = b - A x: x, b read; r written
 static double bytes_residual(long long n, long long e, int t) { return t * (3.0 * n + 2.0 * e) + mask_bytes(n); }
-// damped line sweep: right-hand side and two line factors read, the sweep written;
+// factors of the partitioned line solve: two per node and four per separator and column in
+// FP64, three and three in FP32 (part_factors)
+static double bytes_factors(long long n, int ncol, int P, int t) {
+    const double k = t == 8 ? 2.0 : 3.0;
+    return t * (k * n + (6.0 - k) * std::max(P - 1, 0) * (double)ncol);
+}
+// damped line sweep: right-hand side and line factors read, the sweep written;
 // with the PCG update also q read and the right-hand side written back; a previous
-// iterate read when there is one; the PCG residual read for the final dot products;
-// four factors per separator and column
+// iterate read when there is one; the PCG residual read for the final dot products
 static double bytes_smooth(long long n, int ncol, int P, int t, bool upd, bool xin, bool fin) {
-    const double v = 4.0 + (upd ? 2.0 : 0.0) + (xin ? 1.0 : 0.0) + (fin && !upd ? 1.0 : 0.0);
-    return t * (v * n + 4.0 * std::max(P - 1, 0) * (double)ncol);
+    const double v = 2.0 + (upd ? 2.0 : 0.0) + (xin ? 1.0 : 0.0) + (fin && !upd ? 1.0 : 0.0);
+    return t * v * n + bytes_factors(n, ncol, P, t);
 }
 
 static void prof_close(pf_ctx* ctx, int h) {
@@ -1901,7 +1906,7 @@ static int run_cg(pf_ctx* ctx, int precond, T* x, T* r, T* p, T* p2, T* q, T* z,
         } else if (mg) {
             mg_vcycle<T>(ctx, r, q, z, true, 1);
         } else if (line && pm) {
-            hk = prof_kern<T>(ctx, PF_K_LINE, 0, tb * (6.0 * N + 4.0 * std::max(ps.P - 1, 0) * (double)ncol));
+            hk = prof_kern<T>(ctx, PF_K_LINE, 0, tb * 4.0 * N + bytes_factors(N, ncol, ps.P, (int)sizeof(T)));
             launch_part<T, false>(ctx, ps, ncol, nplanes, plane, r, q, la, lw, lcp, schur, z);
         } else if (line) {
             hk = prof_kern<T>(ctx, PF_K_LINE, 0, tb * 9.0 * N);
