@@ -650,8 +650,8 @@ int pf_grid_set(pf_ctx* ctx, int dim, int geom, const double* ax0, int64_t n0, c
         HIPCK(hipMemcpy(*hf[a], hf32.data(), sizeof(float) * h.size(), hipMemcpyHostToDevice));
         if (dim == 2 && a == 1) {
             for (size_t i = 0; i < h.size(); ++i) {
-                hf32[i] = 1.f / hf32[i];
                 h[i] = 1. / h[i];
+                hf32[i] = (float)h[i];
             }
             if ((rc = dalloc(ctx, &ctx->rhl, h.size()))) return rc;
             if ((rc = dalloc(ctx, &ctx->rhl32, h.size()))) return rc;

@@ -1,8 +1,11 @@
 """FP32 forms: where a quantity is a double rounded once, the results show one rounding."""
+import ctypes as C
+
 import numpy as np
 import pytest
+import torch
 
-from plask_amd.fem import PF_FP32_RELIABLE, PF_FP64, PRECOND_LINE, FemContext
+from plask_amd.fem import PF_FP32_REFINE, PF_FP32_RELIABLE, PF_FP64, PRECOND_LINE, FemContext
 
 pytestmark = pytest.mark.gpu
 
@@ -30,6 +33,35 @@ def test_line_factors_round_once(shape):
     c64, c32 = z64[:-1] / z64[1:], z32[:-1] / z32[1:]
     assert np.abs(z32).min() > 2.0 ** -100
     err = np.abs(c32 / c64 - 1.0)
+    print("largest error %.3f U" % (err.max() / U), flush=True)
+    assert err.max() <= 2.0 * U * (1.0 + 1e-5), err.max() / U
+    c.close()
+
+
+@pytest.mark.parametrize("rows", [1, 2, 5])
+def test_layer_sizes_round_once_2d(rows):
+    """2D operator without in-plane conductivity, kv = 1 and w = 12: next to a row of ones, (A x)_k is
+    that of one layer, 3 (1 / h) times a power of two.  FP64 gives it to 1e-15; FP32 rounds 1 / h and
+    its product with 3: 2 U."""
+    nz = 3001
+    z = np.cumsum(np.r_[0.0, np.random.default_rng(4).uniform(0.05, 2.0, nz - 1)])
+    c = FemContext()
+    c.set_grid([np.array([0.0, 12.0]), z])
+    c.set_coeffs(np.zeros(nz - 1), np.ones(nz - 1))
+    c.set_source(np.zeros(nz - 1))
+    c.set_dirichlet(np.zeros(1, np.int64), np.full(1, 300.0))
+    c.set_launch(16, rows)
+    x = np.zeros((nz, 2))
+    x[::3] = 1.0  # the rows between see one layer each
+    print("layer sizes", rows, flush=True)
+    ref = c.apply(x.ravel()).reshape(nz, 2)
+    xd = torch.tensor(x.ravel(), dtype=torch.float32, device="cuda")
+    y = torch.empty_like(xd)
+    torch.cuda.synchronize()
+    assert c.L.pf_apply(c.h, PF_FP32_REFINE, C.c_void_p(xd.data_ptr()), C.c_void_p(y.data_ptr())) == 0
+    y = y.cpu().numpy().astype(np.float64).reshape(nz, 2)
+    k = np.arange(1, nz - 1)[np.arange(1, nz - 1) % 3 != 0]
+    err = np.abs(y[k] / ref[k] - 1.0)
     print("largest error %.3f U" % (err.max() / U), flush=True)
     assert err.max() <= 2.0 * U * (1.0 + 1e-5), err.max() / U
     c.close()
