@@ -545,7 +545,8 @@ int pf_batch_set(pf_batch* b, int ninst, int cylindrical, const int32_t* n0, con
                  const double* ax1, const double* sh, const double* sv, const int64_t* ndir, const int64_t* dnodes,
                  const double* dvals, const int32_t* jlo, const int32_t* jhi, const double* beta, const double* js);
 /* Times each (block, workgroups) schedule of the persistent kernel on the batch and keeps the
- * fastest; where all instances advance together there is no such choice and one run is timed. */
+ * fastest.  Where all instances advance together there is no such choice: best_seconds is the time
+ * of one run, best_block and best_nwg are the persistent kernel's schedule so far, which stays. */
 int pf_batch_autotune(pf_batch* b, const pf_batch_opts* o, int* best_block, int* best_nwg, double* best_seconds);
 /* Solve every instance from V = Dirichlet values / 0; V_out (concatenated, may be NULL),
  * stats[ninst] (may be NULL), seconds = device time of all launches, with the host's

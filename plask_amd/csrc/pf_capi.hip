@@ -4071,6 +4071,11 @@ static int steps_run(pf_batch* b, const BatchParams& prm, double* seconds, void 
     return PF_OK;
 }
 
+static int batch_cus(const pf_batch* b) {
+    hipDeviceProp_t pr;
+    return hipGetDeviceProperties(&pr, b->device) == hipSuccess ? pr.multiProcessorCount : 256;
+}
+
 extern "C" {
 
 int pf_batch_autotune(pf_batch* b, const pf_batch_opts* o, int* best_block, int* best_nwg, double* best_seconds) {
@@ -4085,29 +4090,31 @@ int pf_batch_autotune(pf_batch* b, const pf_batch_opts* o, int* best_block, int*
         return PF_EINVAL;
     }
     const BatchParams prm = batch_params(o);
-    int props_cu = 256;
-    hipDeviceProp_t pr;
-    if (hipGetDeviceProperties(&pr, b->device) == hipSuccess) props_cu = pr.multiProcessorCount;
+    const int cus = batch_cus(b);
     const int blocks[3] = {256, 512, 1024};
     const int mult[2] = {1, 2};
-    double best = 1e300;
-    int bb = 1024, bn = props_cu;
-    // the step-by-step solve has no such choice: one run gives its time
+    // the step-by-step solve has no such choice: one run gives its time, and the persistent
+    // kernel's schedule stays as it is
     const bool steps = prm.precond == 3 && b->steps.ok;
-    for (int bi = steps ? 2 : 0; bi < 3; ++bi)
-        for (int mi = 0; mi < (steps ? 1 : 2); ++mi) {
-            int nwg = std::min(b->ninst, props_cu * mult[mi]);
-            double t = 0.;
-            int rc = batch_run(b, blocks[bi], nwg, prm, &t, o->progress, o->progress_user);
-            if (rc) return rc;
-            if (t < best) {
-                best = t;
-                bb = blocks[bi];
-                bn = nwg;
+    double best = 1e300;
+    int bb = b->tuned_block ? b->tuned_block : 1024, bn = b->tuned_nwg ? b->tuned_nwg : std::min(b->ninst, cus);
+    if (steps) {
+        if (int rc = batch_run(b, bb, bn, prm, &best, o->progress, o->progress_user)) return rc;
+    } else {
+        for (int block : blocks)
+            for (int m : mult) {
+                const int nwg = std::min(b->ninst, cus * m);
+                double t = 0.;
+                if (int rc = batch_run(b, block, nwg, prm, &t, o->progress, o->progress_user)) return rc;
+                if (t < best) {
+                    best = t;
+                    bb = block;
+                    bn = nwg;
+                }
             }
-        }
-    b->tuned_block = bb;
-    b->tuned_nwg = bn;
+        b->tuned_block = bb;
+        b->tuned_nwg = bn;
+    }
     if (best_block) *best_block = bb;
     if (best_nwg) *best_nwg = bn;
     if (best_seconds) *best_seconds = best;
@@ -4133,15 +4140,12 @@ int pf_batch_solve(pf_batch* b, const pf_batch_opts* o, double* V_out, pf_batch_
         return PF_ESTATE;
     }
     BHIPCK(hipSetDevice(b->device));
-    int props_cu = 256;
-    hipDeviceProp_t pr;
-    if (hipGetDeviceProperties(&pr, b->device) == hipSuccess) props_cu = pr.multiProcessorCount;
     int block = o->block ? o->block : (b->tuned_block ? b->tuned_block : 1024);
     if (block != 256 && block != 512 && block != 1024) {
         b->err = "block must be 256, 512 or 1024";
         return PF_EINVAL;
     }
-    int nwg = o->nwg ? o->nwg : (b->tuned_nwg ? b->tuned_nwg : std::min(b->ninst, props_cu));
+    int nwg = o->nwg ? o->nwg : (b->tuned_nwg ? b->tuned_nwg : std::min(b->ninst, batch_cus(b)));
     if (o->maxloops < 0 || o->loop_budget < 0) {
         b->err = "maxloops and loop_budget must be >= 0";
         return PF_EINVAL;

@@ -83,3 +83,14 @@ def test_steps_progress_and_options():
         st, sp = b.solve(precond=3, **kw)[1], b.solve(precond=2, **kw)[1]
         for a, c in zip(st, sp):
             assert (a["status"], a["loops"], a["iters"]) == (c["status"], c["loops"], c["iters"]), (a, c)
+
+
+def test_autotune_keeps_the_persistent_schedule():
+    """The persistent kernel's tuned schedule outlives an autotune of the step-by-step solve, which
+    has none to choose (600 devices of 4 x 7 nodes: the fewest threads and most workgroups win)."""
+    b = ShockleyBatch([_instance(4, 7, k) for k in range(600)])
+    kw = dict(maxloops=4, maxerr=1e-30)
+    tuned = b.autotune(precond=2, **kw)[:2]
+    steps = b.autotune(precond=3, **kw)
+    print("tuned", tuned, "after the steps", steps[:2], flush=True)
+    assert steps[2] > 0 and steps[:2] == tuned
