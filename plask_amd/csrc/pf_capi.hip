@@ -3095,8 +3095,9 @@ int pf_set_launch(pf_ctx* ctx, int rows, int planes) {
         ctx->KC[0] = ctx->KC[1] = planes;
     } else {
         if (planes < 1) return fail(ctx, PF_EINVAL, "planes >= 1");
-        const int64_t chunks = (ctx->n[1] + planes - 1) / planes;
-        if (chunks > std::max<int64_t>(4096, (ctx->n[1] + 63) / 64) || chunks * ctx->n[0] >= (1LL << 30))
+        // work items of k_apply2d: an index each in 31 bits, a partial sum per block of 256
+        const int64_t items = (ctx->n[1] + planes - 1) / planes * ctx->n[0];
+        if (items >= (1LL << 30) || (size_t)((items + 255) / 256) > ctx->npartials)
             return fail(ctx, PF_EINVAL, "too many blocks for the reduction buffer");
         ctx->KC2 = planes;
     }

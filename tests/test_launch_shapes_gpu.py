@@ -63,6 +63,24 @@ def test_rows_per_thread_2d(rows):
     c.close()
 
 
+@pytest.mark.parametrize("shape", [(4, 10000), (2, 4097), (7, 5001)])
+def test_default_rows_can_be_set_2d(shape):
+    """A tall narrow grid takes one row per thread by default (fewer than 60000 nodes): the same shape
+    set by hand gives the same bits, and so does one of few long marches to the rounding of the operator."""
+    g, axes, kh, kv, dn, c = _problem(shape)
+    print("rows by hand", shape, flush=True)
+    x = np.random.default_rng(1).uniform(-1, 1, g.nnodes)
+    y = c.apply(x)
+    c.set_launch(16, 1)
+    assert np.array_equal(c.apply(x), y)
+    c.set_launch(16, shape[1])
+    assert np.abs(c.apply(x) - y).max() <= 1e-13 * np.abs(y).max()
+    c.set_launch(16, 1)
+    t, st = c.solve(x0=np.full(g.nnodes, 300.0), precision=PF_FP64, rtol=1e-10, precond=PRECOND_LINE)
+    assert st.status == 0 and np.abs(t - 300.0).max() <= 300.0 * 1e-6
+    c.close()
+
+
 @pytest.mark.parametrize("rows,planes", [(2, 1), (3, 1), (4, 1), (4, 7), (31, 40)])
 def test_reductions_over_many_blocks(rows, planes):
     """Grid reductions of one block, of 64 and less (one ticket) and of more (group tickets, the
