@@ -490,12 +490,12 @@ int pf_get_currents(pf_ctx* ctx, double* cur, double* heat);
  * Many independent ElectricalFem2DSolver::compute runs (electr2d.cpp:363-440, junction
  * law beta.hpp:43-46) -- e.g. voltage/temperature sweeps over device variants.  With the
  * multigrid preconditioner all instances advance together, one launch per step over the blocks of
- * those that have not ended, replayed from hipGraphs.  With the line preconditioner, and where a
- * mesh has more than 1032 rows of axis 1 or more than 2049 columns, one persistent kernel: each
- * workgroup takes instances from a largest-first work queue and runs the whole Picard loop.  Either
- * way the loop runs on the device: junction update, preconditioned CG (warm start), currents and
- * loop error.  The reference runs such sweeps as separate processes
- * (gui/plugins/launcher_batch.py:16). */
+ * those that have not ended, replayed from hipGraphs.  With the line preconditioner, where a
+ * mesh has more than 1032 rows of axis 1 or more than 2049 columns, and where the device has no
+ * room for its tables (pf_batch_set_step_memory), one persistent kernel: each workgroup takes
+ * instances from a largest-first work queue and runs the whole Picard loop.  Either way the loop
+ * runs on the device: junction update, preconditioned CG (warm start), currents and loop error.
+ * The reference runs such sweeps as separate processes (gui/plugins/launcher_batch.py:16). */
 typedef struct pf_batch pf_batch;
 
 typedef struct {
@@ -544,6 +544,11 @@ const char* pf_batch_last_error(const pf_batch* b);
 int pf_batch_set(pf_batch* b, int ninst, int cylindrical, const int32_t* n0, const int32_t* n1, const double* ax0,
                  const double* ax1, const double* sh, const double* sv, const int64_t* ndir, const int64_t* dnodes,
                  const double* dvals, const int32_t* jlo, const int32_t* jhi, const double* beta, const double* js);
+/* Device memory that the tables of the multigrid solve in which all instances advance together may
+ * take (about a quarter of what pf_batch_set allocates; bytes < 0: no limit, the default).  The
+ * first multigrid solve allocates them; where they pass the limit or the device has no room for
+ * them, the batch is solved by the persistent kernel. */
+int pf_batch_set_step_memory(pf_batch* b, int64_t bytes);
 /* Times each (block, workgroups) schedule of the persistent kernel on the batch and keeps the
  * fastest.  Where all instances advance together there is no such choice: best_seconds is the time
  * of one run, best_block and best_nwg are the persistent kernel's schedule so far, which stays. */

@@ -39,6 +39,7 @@ def _decl(L):
     L.pf_batch_last_error.argtypes = [P]
     L.pf_batch_last_error.restype = C.c_char_p
     L.pf_batch_set.argtypes = [P, I, I, P, P, P, P, P, P, P, P, P, P, P, P, P]
+    L.pf_batch_set_step_memory.argtypes = [P, C.c_int64]
     L.pf_batch_autotune.argtypes = [P, C.POINTER(BatchOpts), C.POINTER(I), C.POINTER(I), C.POINTER(C.c_double)]
     L.pf_batch_solve.argtypes = [P, C.POINTER(BatchOpts), P, P, C.POINTER(C.c_double)]
     L.pf_batch_conductivities.argtypes = [P, P, P]
@@ -98,6 +99,11 @@ class ShockleyBatch:
         progress: print a line at every report."""
         return BatchOpts(maxloops, maxit, maxerr, rtol, 1 if stable else 0, block, nwg, int(precond),
                          int(loop_budget), _PRINT_PROGRESS if progress else _NO_PROGRESS, None)
+
+    def set_step_memory(self, nbytes):
+        """Device bytes that the tables of the multigrid solve may take (negative: no limit).  A batch
+        whose tables need more is solved by the persistent kernel."""
+        self._ck(self.L.pf_batch_set_step_memory(self.h, int(nbytes)), "pf_batch_set_step_memory")
 
     def autotune(self, **kw):
         o = self.opts(**kw)

@@ -10,11 +10,13 @@
 #include <algorithm>
 #include <chrono>
 #include <cmath>
+#include <cstdint>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
 #include <map>
 #include <mutex>
+#include <new>
 #include <string>
 #include <type_traits>
 #include <vector>
@@ -3355,9 +3357,11 @@ int pf_time_apply(pf_ctx* ctx, int precision, int reps, double* seconds) {
 // ===========================================================================
 // Batched 2D Shockley solver (persistent kernel over a work queue)
 // ===========================================================================
-// Tables and launch shapes of the step-by-step batch solve
+// Tables and launch shapes of the step-by-step batch solve, built by the first multigrid solve
 struct BatchSteps {
-    bool ok = false;
+    bool tried = false, ok = false;  // built at all, and in use
+    size_t limit = SIZE_MAX, bytes = 0;  // device bytes allowed and taken
+    std::vector<void*> allocs;
     BsArgs args{};
     int levels = 0;  // levels outside the tail kernel, at most
     struct Map {
@@ -3372,6 +3376,14 @@ struct BatchSteps {
     hipGraphExec_t g_first = nullptr, g_loop = nullptr, g_iter = nullptr, g_start = nullptr, g_end = nullptr,
                    g_cur = nullptr;
     BatchParams prm{};
+};
+
+// What the tables are built from, kept from pf_batch_set until then
+struct BatchHost {
+    std::vector<BatchInst> inst;
+    std::vector<BatchLevel> levs;
+    std::vector<int> order;  // largest instances first
+    std::vector<uint64_t> mask, lmask;
 };
 
 struct pf_batch {
@@ -3393,8 +3405,9 @@ struct pf_batch {
     unsigned int* hfin = nullptr;  // pinned: instances finished, read between launches
     // multigrid levels of all instances (pools described by BatchLevel)
     BatchMg mg{};
-    // all instances step by step (batch_steps.hpp), where the meshes allow it
+    // all instances step by step (batch_steps.hpp), where the meshes and the memory allow it
     BatchSteps steps;
+    BatchHost host;
     std::vector<long long> node_off;
     int tuned_block = 0, tuned_nwg = 0;
     std::vector<void*> allocs;
@@ -3426,6 +3439,32 @@ static void steps_drop(BatchSteps& S) {
     }
 }
 
+// Device memory of the step tables; STEPS_NO_ROOM where the limit or the device does not hold it
+constexpr int STEPS_NO_ROOM = 1;
+template <typename T> static int steps_alloc(pf_batch* b, T** ptr, size_t count) {
+    BatchSteps& S = b->steps;
+    const size_t bytes = sizeof(T) * std::max<size_t>(count, 1);
+    if (bytes > S.limit - S.bytes) return STEPS_NO_ROOM;
+    const hipError_t e = hipMalloc((void**)ptr, bytes);
+    if (e == hipErrorOutOfMemory) {
+        (void)hipGetLastError();
+        return STEPS_NO_ROOM;
+    }
+    BHIPCK(e);
+    S.allocs.push_back((void*)*ptr);
+    S.bytes += bytes;
+    return PF_OK;
+}
+
+static void steps_free(BatchSteps& S) {
+    steps_drop(S);
+    for (void* p : S.allocs) hipFree(p);
+    S.allocs.clear();
+    S.bytes = 0;
+    if (S.count) hipHostFree(S.count);
+    S.count = nullptr;
+}
+
 __global__ void k_copy_d(long long n, const double* __restrict__ a, double* __restrict__ b) {
     for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x)
         b[i] = a[i];
@@ -3436,10 +3475,12 @@ __global__ void k_copy_d(long long n, const double* __restrict__ a, double* __re
 // separator scan takes (n1 > 1032; the walk of one thread per column would be the chain of
 // latencies this solve avoids) or whose element rows do not fit k_bs_coarsen's LDS (n0 > 2049)
 // stay with the persistent kernel.
-static int steps_build(pf_batch* b, const std::vector<BatchInst>& inst, const std::vector<BatchLevel>& levs,
-                       const std::vector<int>& order, const std::vector<uint64_t>& mask,
-                       const std::vector<uint64_t>& lmask) {
+static int steps_build(pf_batch* b) {
     BatchSteps& S = b->steps;
+    const std::vector<BatchInst>& inst = b->host.inst;
+    const std::vector<BatchLevel>& levs = b->host.levs;
+    const std::vector<int>& order = b->host.order;
+    const std::vector<uint64_t>&mask = b->host.mask, &lmask = b->host.lmask;
     const int ninst = b->ninst;
     long long widest = 0;
     for (const BatchInst& I : inst) {
@@ -3477,12 +3518,14 @@ static int steps_build(pf_batch* b, const std::vector<BatchInst>& inst, const st
             std::vector<unsigned char>& fx = fixed[l > 0];
             L.seg = (long long)fx.size();
             fx.resize(fx.size() + (size_t)L.P * L.n0, 0);
-            for (int k = 0; k < L.n1; ++k)
-                for (int c = 0; c < L.n0; ++c) {
-                    const long long bit = L.mask + (long long)k * L.n0 + c;
-                    if ((mk[bit >> 6] >> (bit & 63)) & 1ull)
-                        fx[L.seg + (size_t)(k / BS_M) * L.n0 + c] |= (unsigned char)(1u << (k % BS_M));
-                }
+            const long long end = L.mask + (long long)L.n0 * L.n1;
+            for (long long bit = L.mask; bit < end; ++bit) {  // from one fixed node to the next
+                const uint64_t w = mk[bit >> 6] >> (bit & 63);
+                bit = w ? bit + __builtin_ctzll(w) : (bit | 63);
+                if (!w || bit >= end) continue;
+                const int k = (int)((bit - L.mask) / L.n0), c = (int)((bit - L.mask) % L.n0);
+                fx[L.seg + (size_t)(k / BS_M) * L.n0 + c] |= (unsigned char)(1u << (k % BS_M));
+            }
             S.sweep_lds = std::max(S.sweep_lds, sizeof(double) * (size_t)part_lds_values(L.P, L.CB, BS_T));
             S.up_lds = std::max(S.up_lds, sizeof(double) * (size_t)bs_up_lds(L.n1, L.P, L.CB));
             tab.push_back(L);
@@ -3507,7 +3550,7 @@ static int steps_build(pf_batch* b, const std::vector<BatchInst>& inst, const st
     auto put = [&](auto** dst, const auto& v) -> int {
         using T = typename std::remove_reference<decltype(v[0])>::type;
         typename std::remove_const<T>::type* d = nullptr;
-        if (int r = balloc(b, &d, v.size())) return r;
+        if (int r = steps_alloc(b, &d, v.size())) return r;
         if (!v.empty()) BHIPCK(hipMemcpy(d, v.data(), sizeof(T) * v.size(), hipMemcpyHostToDevice));
         *dst = d;
         return PF_OK;
@@ -3555,16 +3598,20 @@ static int steps_build(pf_batch* b, const std::vector<BatchInst>& inst, const st
     int *dl0 = nullptr, *dt = nullptr;
     long long* dp = nullptr;
     if ((rc = put(&dl, tab)) || (rc = put(&dl0, lev0)) || (rc = put(&dt, tail)) || (rc = put(&dp, part)) ||
-        (rc = balloc(b, &A.schur, schur)) || (rc = balloc(b, &A.partials, npart)) || (rc = balloc(b, &A.st, ninst)) ||
-        (rc = balloc(b, &A.PB, b->N)) || (rc = balloc(b, &A.count, 2)))
+        (rc = steps_alloc(b, &A.schur, schur)) || (rc = steps_alloc(b, &A.partials, npart)) || (rc = steps_alloc(b, &A.st, ninst)) ||
+        (rc = steps_alloc(b, &A.PB, b->N)) || (rc = steps_alloc(b, &A.count, 2)))
         return rc;
     unsigned char* dfx[2] = {nullptr, nullptr};
     double *ea[2], *eb[2];
     for (int c = 0; c < 2; ++c)
-        if ((rc = put(&dfx[c], fixed[c])) || (rc = balloc(b, &ea[c], c ? nelem : b->E)) ||
-            (rc = balloc(b, &eb[c], c ? nelem : b->E)))
+        if ((rc = put(&dfx[c], fixed[c])) || (rc = steps_alloc(b, &ea[c], c ? nelem : b->E)) ||
+            (rc = steps_alloc(b, &eb[c], c ? nelem : b->E)))
             return rc;
-    BHIPCK(hipHostMalloc((void**)&S.count, 2 * sizeof(int), hipHostMallocDefault));
+    if (hipHostMalloc((void**)&S.count, 2 * sizeof(int), hipHostMallocDefault) != hipSuccess) {
+        (void)hipGetLastError();
+        S.count = nullptr;
+        return STEPS_NO_ROOM;
+    }
     A.inst = b->dinst;
     A.lev = dl;
     A.lev0 = dl0;
@@ -3582,6 +3629,23 @@ static int steps_build(pf_batch* b, const std::vector<BatchInst>& inst, const st
     A.cur = b->cur;
     A.stats = b->dstats;
     S.ok = true;
+    return PF_OK;
+}
+
+// The step tables, once: a batch that they do not fit beside stays with the persistent kernel.
+static int steps_ready(pf_batch* b) {
+    BatchSteps& S = b->steps;
+    if (S.tried) return PF_OK;
+    int rc;
+    try {
+        rc = steps_build(b);
+    } catch (const std::bad_alloc&) {  // host memory
+        rc = STEPS_NO_ROOM;
+    }
+    if (!S.ok) steps_free(S);
+    if (rc && rc != STEPS_NO_ROOM) return rc;
+    S.tried = true;
+    b->host = BatchHost{};
     return PF_OK;
 }
 
@@ -3615,8 +3679,7 @@ void pf_batch_destroy(pf_batch* b) {
     hipStreamSynchronize(b->stream);
     if (b->graph) hipGraphExecDestroy(b->graph);
     if (b->graph_init) hipGraphExecDestroy(b->graph_init);
-    steps_drop(b->steps);
-    if (b->steps.count) hipHostFree(b->steps.count);
+    steps_free(b->steps);
     for (void* p : b->allocs) hipFree(p);
     if (b->hfin) hipHostFree(b->hfin);
     hipStreamDestroy(b->stream);
@@ -3814,7 +3877,18 @@ int pf_batch_set(pf_batch* b, int ninst, int cylindrical, const int32_t* n0, con
     BHIPCK(hipMemcpy(b->kv0, sv, sizeof(double) * E, hipMemcpyHostToDevice));
     BHIPCK(hipMemcpy(b->dmask, mask.data(), sizeof(uint64_t) * mask.size(), hipMemcpyHostToDevice));
     BHIPCK(hipMemcpy(b->x0, x0.data(), sizeof(double) * N, hipMemcpyHostToDevice));
-    return steps_build(b, inst, levs, order, mask, lmask);
+    b->host = BatchHost{std::move(inst), std::move(levs), std::move(order), std::move(mask), std::move(lmask)};
+    return PF_OK;
+}
+
+int pf_batch_set_step_memory(pf_batch* b, int64_t bytes) {
+    if (!b) return PF_EINVAL;
+    if (b->steps.tried) {
+        b->err = "pf_batch_set_step_memory comes before the first multigrid solve";
+        return PF_ESTATE;
+    }
+    b->steps.limit = bytes < 0 ? SIZE_MAX : (size_t)bytes;
+    return PF_OK;
 }
 
 }  // extern "C"
@@ -3879,8 +3953,11 @@ static int steps_run(pf_batch* b, const BatchParams& prm, double* seconds, void 
 
 static int batch_run(pf_batch* b, int block, int nwg, const BatchParams& prm, double* seconds,
                      void (*progress)(int, int, int, double, void*), void* user) {
-    if (prm.precond == 3 && b->steps.ok) return steps_run(b, prm, seconds, progress, user);
     int rc;
+    if (prm.precond == 3) {
+        if ((rc = steps_ready(b))) return rc;
+        if (b->steps.ok) return steps_run(b, prm, seconds, progress, user);
+    }
     if (b->graphs) {
         if (!b->graph_init && (rc = batch_capture(b, &b->graph_init, [&] { batch_launch_init(b); }))) return rc;
         if (!b->graph || b->graph_block != block || b->graph_nwg != nwg || !same_prm(b->graph_prm, prm)) {
@@ -4096,6 +4173,8 @@ int pf_batch_autotune(pf_batch* b, const pf_batch_opts* o, int* best_block, int*
     const int mult[2] = {1, 2};
     // the step-by-step solve has no such choice: one run gives its time, and the persistent
     // kernel's schedule stays as it is
+    if (prm.precond == 3)
+        if (int rc = steps_ready(b)) return rc;
     const bool steps = prm.precond == 3 && b->steps.ok;
     double best = 1e300;
     int bb = b->tuned_block ? b->tuned_block : 1024, bn = b->tuned_nwg ? b->tuned_nwg : std::min(b->ninst, cus);

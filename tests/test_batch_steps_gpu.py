@@ -3,9 +3,11 @@ launch shapes change: meshes without coarse levels, rows and columns around a se
 block, one and two separators per scan lane, lines too long for the scan (persistent kernel)."""
 import numpy as np
 import pytest
+import torch
 
 import oracle as O
 from plask_amd.batch import PROGRESS, ShockleyBatch
+from plask_amd.fem import FemError
 
 pytestmark = pytest.mark.gpu
 
@@ -94,3 +96,46 @@ def test_autotune_keeps_the_persistent_schedule():
     steps = b.autotune(precond=3, **kw)
     print("tuned", tuned, "after the steps", steps[:2], flush=True)
     assert steps[2] > 0 and steps[:2] == tuned
+
+
+def test_tables_come_with_the_first_multigrid_solve():
+    """The tables of the step-by-step solve are built by the first solve that uses them, which takes
+    more than five values per node.  Where they pass the limit the persistent kernel solves the batch:
+    no memory beyond what its line-preconditioned solve has taken (the runtime's scratch memory for
+    that kernel and stream), the same statuses, and potentials to the conditioning of the systems
+    times the tolerance (1e-8, as above)."""
+    kw = dict(maxloops=2, maxerr=1e-30, rtol=1e-13)
+    sizes = [(150 + 37 * k, 410 + 60 * k) for k in range(6)]
+    insts = [_instance(n0, n1, k) for k, (n0, n1) in enumerate(sizes)]
+    nodes = sum(n0 * n1 for n0, n1 in sizes)
+    print("step tables", sizes, flush=True)
+
+    def used():
+        torch.cuda.synchronize()
+        free, total = torch.cuda.mem_get_info()
+        return total - free
+
+    def growth(batch):
+        batch.solve(precond=2, maxloops=1, maxit=20)
+        at = used()
+        V, stats, _t = batch.solve(precond=3, **kw)
+        values = (used() - at) / (8.0 * nodes)
+        print("grows by %.2f values per node" % values, flush=True)
+        return V, stats, values
+
+    b = ShockleyBatch(insts)
+    V, stats, values = growth(b)
+    assert values > 5
+    with pytest.raises(FemError, match="before the first multigrid solve"):
+        b.set_step_memory(-1)
+    for limit in (0, 3 * 8 * nodes):  # none of the tables, and some of them
+        p = ShockleyBatch(insts)
+        p.set_step_memory(limit)
+        Vp, sp, values = growth(p)
+        assert values < 1
+        for v, q, s, r in zip(V, Vp, stats, sp):
+            assert s["status"] == r["status"] and s["loops"] == r["loops"], (s, r)
+            assert np.abs(v - q).max() <= 1e-8 * np.abs(v).max()
+        tuned = p.autotune(precond=3, **kw)
+        assert tuned[2] > 0
+        p.close()
