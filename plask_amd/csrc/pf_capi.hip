@@ -149,6 +149,7 @@ struct pf_ctx {
     // cached graphs of one chunk of iterations
     hipGraphExec_t graph64 = nullptr, graph32 = nullptr;
     hipGraphExec_t graph_end[2] = {nullptr, nullptr};  // the last 2 iterations (run_cg)
+    bool end_ran[2] = {false, false};                  // they have run once, as plain launches
     int graph_chunk[2] = {0, 0}, graph_key[2] = {-1, -1};  // what graph64 / graph32 hold
     bool prec32 = false;  // FP64 PCG with the preconditioner applied in FP32 (PF_FP64_PREC32)
 
@@ -249,6 +250,7 @@ static void drop_graphs(pf_ctx* ctx) {
     }
     ctx->graph64 = ctx->graph32 = nullptr;
     ctx->graph_key[0] = ctx->graph_key[1] = -1;
+    ctx->end_ran[0] = ctx->end_ran[1] = false;
 }
 
 // Profiled chunks: prof_open records a start event for one kernel category (returns a
@@ -2007,23 +2009,32 @@ static int run_cg(pf_ctx* ctx, int precond, T* x, T* r, T* p, T* p2, T* q, T* z,
             if (*gcache) hipGraphExecDestroy(*gcache);
             if (*gend) hipGraphExecDestroy(*gend);
             *gcache = *gend = nullptr;
+            ctx->end_ran[gi] = false;
             if (int rc = capture(gcache, chunk)) return rc;
             ctx->graph_chunk[gi] = chunk;
             ctx->graph_key[gi] = key;
         }
         // Multigrid iterations past the stop are ~30 launches each that only find the flag (2.3 us
         // each): where the mean reduction per iteration so far says that 2 iterations reach the
-        // stop, a graph of 2 runs instead of the chunk of 4 (25 x 19 x 37 nodes, 13 iterations;
-        // two replays of such a graph in place of the chunk cost 10 us more per chunk).
+        // stop, 2 run instead of the chunk of 4, the first time as plain launches and from then on
+        // as a graph of their own (25 x 19 x 37 nodes, 13 iterations: the first solve of a grid
+        // 3.11 ms, 3.29 with the capture in it; replays 1.69 ms, 1.70 with plain launches every
+        // time; two replays of such a graph in place of the chunk cost 10 us more per chunk).
         auto near_end = [&]() {
             const PcgState& s = *ctx->hst;
             const double per_iter = s.iters > 0 ? std::log(s.rr0 / s.rr) / s.iters : 0.;
             return mg && chunk == 4 && per_iter > 0. && std::log(s.rr / s.stop2) <= 2. * per_iter;
         };
         for (bool end = false;; end = near_end()) {
-            if (end && !*gend)
-                if (int rc = capture(gend, 2)) return rc;
-            HIPCK(hipGraphLaunch(end ? *gend : *gcache, ctx->stream));
+            if (end && !ctx->end_ran[gi]) {
+                for (int c = 0; c < 2; ++c) one_iter(c);
+                HIPCK(hipGetLastError());
+                ctx->end_ran[gi] = true;
+            } else {
+                if (end && !*gend)
+                    if (int rc = capture(gend, 2)) return rc;
+                HIPCK(hipGraphLaunch(end ? *gend : *gcache, ctx->stream));
+            }
             HIPCK(hipMemcpyAsync(ctx->hst, ctx->st, sizeof(PcgState), hipMemcpyDeviceToHost, ctx->stream));
             HIPCK(hipStreamSynchronize(ctx->stream));
             if (ctx->hst->done) break;

@@ -133,3 +133,23 @@ def test_last_iterations_in_a_short_graph(rtol):
     b, sb = c.solve(rtol=rtol, check_every=2, **kw)
     assert sa.iters == sb.iters and np.array_equal(a, b)
     c.close()
+
+
+def test_first_solves_of_a_grid():
+    """The short last part of a solve runs as plain launches, is captured and is replayed in the first
+    three solves after a grid is set: all have the iterations and bits of checks every 2."""
+    g, axes, kh, kv, dn, c = _problem((17, 15, 24))
+    kw = dict(x0=np.full(g.nnodes, 300.0), precision=PF_FP64, precond=PRECOND_MG, rtol=1e-9)
+    q = np.random.default_rng(3).uniform(0, 1e16, g.nelems)
+    print("first solves", flush=True)
+    c.set_source(q)
+    ref, sr = c.solve(check_every=2, **kw)
+    for _ in range(2):
+        c.set_grid(axes)
+        c.set_coeffs(kh, kv)
+        c.set_source(q)
+        c.set_dirichlet(dn, np.full(len(dn), 300.0))
+        for _ in range(4):
+            t, st = c.solve(**kw)
+            assert st.iters == sr.iters and np.array_equal(t, ref)
+    c.close()
