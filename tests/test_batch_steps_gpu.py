@@ -6,6 +6,7 @@ import pytest
 import torch
 
 import oracle as O
+from plask_amd import workloads
 from plask_amd.batch import PROGRESS, ShockleyBatch
 from plask_amd.fem import FemError
 
@@ -139,3 +140,63 @@ def test_tables_come_with_the_first_multigrid_solve():
         tuned = p.autotune(precond=3, **kw)
         assert tuned[2] > 0
         p.close()
+
+
+# seeds of stiff devices (conductivities over seven decades) whose CG stops with a true residual
+# above its recursive one, so that the loop asks for a second run
+STIFF = (3000, 3005, 3008, 3009, 3011)
+
+
+def _stiff_and_easy():
+    stiff = [workloads.shockley_cyl_batch(n_inst=1, seed0=s, nr_range=(12, 40), nz_range=(30, 70))[0] for s in STIFF]
+    easy = [_instance(20 + 3 * k, 40 + 5 * k, k) for k in range(4)]
+    insts, is_stiff = [], []
+    for k in range(5):  # next to each other in the launches
+        for group, name in ((stiff, True), (easy, False)):
+            if k < len(group):
+                insts.append(group[k])
+                is_stiff.append(name)
+    return insts, np.array(is_stiff)
+
+
+@pytest.mark.parametrize("loops", [1, 4])
+def test_second_runs_of_stiff_instances(loops):
+    """CG starts once more from the true residual where that has not followed the recursive one: in
+    the first loop for the stiff devices and for no easy one, while the others wait.  Restarts as in
+    the persistent kernel in the first loop (later ones start from potentials that differ by rounding),
+    statuses and loops as with the line preconditioner, potentials as the oracle's (1e-8, as above)."""
+    insts, stiff = _stiff_and_easy()
+    kw = dict(maxloops=loops, maxerr=1e-30, rtol=1e-12)
+    print("second runs", loops, flush=True)
+    b = ShockleyBatch(insts)
+    p = ShockleyBatch(insts)
+    p.set_step_memory(0)  # the persistent kernel
+    line = b.solve(precond=2, **kw)[1]
+    for _ in range(2):  # the second solve replays the graphs on the state of the first
+        V, stats, _t = b.solve(precond=3, **kw)
+        restarts = np.array([s["restarts"] for s in stats])
+        print("restarts", restarts, flush=True)
+        assert (restarts[stiff] > 0).all()
+        if loops == 1:
+            assert (restarts[~stiff] == 0).all()
+            assert restarts.tolist() == [s["restarts"] for s in p.solve(precond=3, **kw)[1]]
+        for q, v, s, r in zip(insts, V, stats, line):
+            Vr = _oracle(q, loops)[0]
+            assert (s["status"], s["loops"]) == (r["status"], r["loops"]) == (2, loops)
+            assert np.abs(v - Vr).max() <= 1e-8 * np.abs(Vr).max(), (np.abs(v - Vr).max(), s)
+
+
+def test_steps_as_plain_launches(monkeypatch):
+    """Without graphs (as under a tracing profiler, whose environment turns them off) the same bits."""
+    insts, _ = _stiff_and_easy()
+    kw = dict(maxloops=4, maxerr=1e-30, rtol=1e-12, precond=3)
+    print("plain launches", flush=True)
+    V, stats, _t = ShockleyBatch(insts).solve(**kw)
+    monkeypatch.setenv("ROCPROF_OUTPUT_PATH", "x")  # read when a batch is created
+    p = ShockleyBatch(insts)
+    monkeypatch.delenv("ROCPROF_OUTPUT_PATH")
+    for _ in range(2):
+        Vp, sp, _t = p.solve(**kw)
+        assert stats == sp
+        for v, q in zip(V, Vp):
+            assert np.array_equal(v, q)
