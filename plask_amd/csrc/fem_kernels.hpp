@@ -1268,7 +1268,8 @@ __global__ void k_line_setup2d(Axes2<double> g, const double* __restrict__ kh, c
 // separators, or one thread's walk for lines of more than 128 separators; part_solve).
 // Stored per node:
 //   interior plane: la = coupling to the previous interior plane (0 on the
-//     first), lw = LDL^T pivot inverse, lcp = c' (0 on the last);
+//     first), lw = LDL^T pivot inverse, lcp = c' (0 on the last; FP32 only, FP64
+//     forms it from la and lw, see part_factors);
 //   separator: la = coupling to the plane below, lcp = coupling to the plane
 //     above (lw holds the diagonal, read only here).
 // schur[(0|1|2)(P-1) + j][col] = Thomas factors (a, w, c') of S.
@@ -1336,7 +1337,7 @@ __device__ inline void part_factor_segment(int col, int s, int ncol, int n, int 
             const double cp = last ? 0. : c * w;
             la[node] = T(a);
             lw[node] = T(w);
-            lcp[node] = T(cp);
+            if (sizeof(T) == 4) lcp[node] = T(cp);
             cprev = c;
             cpprev = cp;
         }
