@@ -93,17 +93,16 @@ static int gridn(long long n, int threads = 256, int cap = 8192) {
 // ---------------------------------------------------------------------------
 // convolution dispatch
 // ---------------------------------------------------------------------------
-// Launch shape of k_conv3: output channels per block (16 NT) and x rows per wave (ZT x YT).
-// Larger blocks reuse weights and halo more; smaller ones give a small volume enough blocks
-// for the 256 CUs.
+// Launch shape of k_conv3: x rows per wave (ZT x YT).  Larger blocks reuse weights and halo
+// more; smaller ones give a small volume enough blocks for the 256 CUs.
 static long long conv_blocks(const Vol& o, int ZT, int YT) {
     return (long long)ceil_div(o.nx, 16) * ceil_div(o.ny, 2 * YT) * ceil_div(o.nz, 2 * ZT);
 }
 
-template <int CIN, int NT, int ZT, int YT, bool UP, bool RELU>
+template <int CIN, int ZT, int YT, bool UP, bool RELU>
 static void conv_launch(pf_net* net, const Vol& o, const bf16* in, const bf16* w, const float* bias, const bf16* skip,
                         bf16* out, int cout) {
-    hipLaunchKernelGGL((k_conv3<CIN, NT, ZT, YT, UP, RELU>), dim3((unsigned)conv_blocks(o, ZT, YT), cout / (16 * NT)),
+    hipLaunchKernelGGL((k_conv3<CIN, ZT, YT, UP, RELU>), dim3((unsigned)conv_blocks(o, ZT, YT), cout / (16 * CONV_NT)),
                        dim3(256), 0, net->stream, o, in, w, bias, skip, out, cout);
 }
 
@@ -111,16 +110,13 @@ template <int CIN, bool UP, bool RELU>
 static void conv(pf_net* net, const Vol& o, const bf16* in, const bf16* w, const float* bias, const bf16* skip,
                  bf16* out, int cout) {
     constexpr long long MINB = 512;  // blocks wanted (256: 2 % slower, 1024: 2 %)
-    const long long b24 = conv_blocks(o, 2, 4), b22 = conv_blocks(o, 2, 2);
-    const int n4 = cout / 64, n2 = cout / 32;
-    if (CIN >= 32 && n4 && b24 * n4 >= MINB) {
-        if constexpr (CIN >= 32) conv_launch<CIN, 4, 2, 4, UP, RELU>(net, o, in, w, bias, skip, out, cout);
-    } else if (b24 * n2 >= MINB) {
-        conv_launch<CIN, 2, 2, 4, UP, RELU>(net, o, in, w, bias, skip, out, cout);
-    } else if (UP || b22 * n2 >= MINB) {
-        conv_launch<CIN, 2, 2, 2, UP, RELU>(net, o, in, w, bias, skip, out, cout);
+    const int n = cout / (16 * CONV_NT);
+    if (conv_blocks(o, 2, 4) * n >= MINB) {
+        conv_launch<CIN, 2, 4, UP, RELU>(net, o, in, w, bias, skip, out, cout);
+    } else if (UP || conv_blocks(o, 2, 2) * n >= MINB) {
+        conv_launch<CIN, 2, 2, UP, RELU>(net, o, in, w, bias, skip, out, cout);
     } else {
-        if constexpr (!UP) conv_launch<CIN, 2, 1, 1, UP, RELU>(net, o, in, w, bias, skip, out, cout);
+        if constexpr (!UP) conv_launch<CIN, 1, 1, UP, RELU>(net, o, in, w, bias, skip, out, cout);
     }
 }
 

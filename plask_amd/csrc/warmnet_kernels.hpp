@@ -27,7 +27,8 @@ struct Vol {
 __device__ __forceinline__ float b2f(bf16 v) { return (float)v; }
 __device__ __forceinline__ bf16 f2b(float v) { return (bf16)v; }
 
-// tap t = (dz + 1) * 9 + (dy + 1) * 3 + (dx + 1); tap 26 - t is the mirrored offset
+// Taps: t = (dz + 1) * 9 + (dy + 1) * 3 + (dx + 1); tap 26 - t is the mirrored offset.
+//
 // Bricks of output voxels: every convolution kernel works on bricks of 16 x 2 YT x 2 ZT
 // voxels, whose input (with a halo of one voxel) is staged through LDS once and read from
 // there by all 27 taps.
@@ -92,7 +93,7 @@ __device__ __forceinline__ void stage_input(const Vol& iv, const bf16* __restric
 }
 
 // Output-stationary 3x3x3 convolution.  A block of 4 waves takes a brick of 16 x 2 YT x 2 ZT
-// voxels and 16 NT output channels; a wave takes ZT x YT of the brick's x rows (16 voxels
+// voxels and 16 CONV_NT output channels; a wave takes ZT x YT of the brick's x rows (16 voxels
 // each) and keeps their accumulators in registers.  Input channels go in chunks of 32
 // through LDS; per chunk and x offset the wave holds all the input rows its outputs touch
 // ((ZT + 2) x (YT + 2), or half of that with the upsampling, where several taps of one
@@ -102,13 +103,18 @@ __device__ __forceinline__ void stage_input(const Vol& iv, const bf16* __restric
 // What bounds it: the matrix cores and the instructions around them.  The earlier kernel
 // (one wave per 16 voxels, both operands from global memory for every tap) was held by L1:
 // each input value was fetched 27 times and all weights once per 16 voxels.  At 64 x 64 x
-// 128 voxels, before and after: 64 -> 32 channels upsampled 523 -> 59 us (1.0 PFLOP/s),
-// 128 -> 64 upsampled 228 -> 46 us, 8 -> 32 30 -> 21 us, 32 -> 64 backward data 247 -> 91 us.
-template <int CIN, int NT, int ZT, int YT, bool UP, bool RELU>
+// 128 voxels, before and after: 64 -> 32 channels upsampled 523 -> 65 us (0.89 PFLOP/s),
+// 128 -> 64 upsampled 228 -> 42 us, 8 -> 32 30 -> 22 us, 32 -> 64 backward data 247 -> 82 us.
+// 32 output channels per block: with 64 the last of these took 88 us, a training step of 128 x 128
+// x 256 voxels 4.45 instead of 4.30 ms, and no size gained (twice the accumulators: one wave per
+// SIMD instead of two).
+constexpr int CONV_NT = 2;
+template <int CIN, int ZT, int YT, bool UP, bool RELU>
 __global__ __launch_bounds__(256) void k_conv3(Vol o, const bf16* __restrict__ in, const bf16* __restrict__ w,
                                                const float* __restrict__ bias, const bf16* __restrict__ skip,
                                                bf16* __restrict__ out, int cout) {
     using H = Halo<UP, ZT, YT>;
+    constexpr int NT = CONV_NT;
     constexpr int CK = CIN < 32 ? CIN : 32;
     __shared__ __align__(16) unsigned char tile[H::N * CK * 2];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
