@@ -601,8 +601,19 @@ static int tile_planes(int BY, int n1, int n2, int kmax) {
 }
 
 // 2D: rows of axis 1 per thread: long marches reuse the neighbouring rows, short ones give the
-// small grids enough waves (and keep n0 * chunks in 31 bits).  A multigrid solve of 200 x 400
-// nodes takes 1.97 ms with these (1 row on its coarse levels, 2 on the solve grid).
+// small grids enough waves (and keep n0 * chunks in 31 bits).  60 iterations with the line
+// preconditioner in FP64, ms (FP32 has its best at the same or the next longer march):
+//   nodes      1 row    2      4      8     16
+//     58 e3    1.14   1.17   1.21   1.34   1.62
+//     80 e3    1.29   1.22   1.28   1.38   1.67
+//    240 e3    2.01   1.84   1.80   1.93   2.18
+//    600 e3    2.72   2.44   2.30   2.33   2.34
+//      1 e6    3.54   3.16   2.75   2.61   2.63
+//      2 e6    8.26   7.63   6.84   6.60   6.39
+//    4.1 e6    37.0   35.5   33.7   33.1   32.7
+// The unrolling by 4 (240 registers, 2 waves per SIMD in the fused FP64 form) is the better one on
+// every grid that takes it.  At 2 e6 the residuals of the FP32 multigrid have the last word: their
+// plain product takes 8.7 us with 8 rows and 9.4 with 16.
 static int rows2d(long long n0, long long n1) {
     const long long N = n0 * n1;
     int KC = N >= 4000000 ? 16 : N >= 1000000 ? 8 : N >= 240000 ? 4 : N >= 60000 ? 2 : 1;
