@@ -3,9 +3,9 @@ launch shapes change: meshes without coarse levels, rows and columns around a se
 block, one and two separators per scan lane, lines too long for the scan (persistent kernel)."""
 import numpy as np
 import pytest
-import torch
 
 import oracle as O
+from hip_runtime import memory_used
 from plask_amd import workloads
 from plask_amd.batch import PROGRESS, ShockleyBatch
 from plask_amd.fem import FemError
@@ -111,16 +111,11 @@ def test_tables_come_with_the_first_multigrid_solve():
     nodes = sum(n0 * n1 for n0, n1 in sizes)
     print("step tables", sizes, flush=True)
 
-    def used():
-        torch.cuda.synchronize()
-        free, total = torch.cuda.mem_get_info()
-        return total - free
-
     def growth(batch):
         batch.solve(precond=2, maxloops=1, maxit=20)
-        at = used()
+        at = memory_used()
         V, stats, _t = batch.solve(precond=3, **kw)
-        values = (used() - at) / (8.0 * nodes)
+        values = (memory_used() - at) / (8.0 * nodes)
         print("grows by %.2f values per node" % values, flush=True)
         return V, stats, values
 

@@ -1,10 +1,8 @@
 """FP32 forms: where a quantity is a double rounded once, the results show one rounding."""
-import ctypes as C
-
 import numpy as np
 import pytest
-import torch
 
+from hip_runtime import DeviceArray
 from plask_amd.fem import PF_FP32_REFINE, PF_FP32_RELIABLE, PF_FP64, PRECOND_LINE, FemContext
 
 pytestmark = pytest.mark.gpu
@@ -55,11 +53,11 @@ def test_layer_sizes_round_once_2d(rows):
     x[::3] = 1.0  # the rows between see one layer each
     print("layer sizes", rows, flush=True)
     ref = c.apply(x.ravel()).reshape(nz, 2)
-    xd = torch.tensor(x.ravel(), dtype=torch.float32, device="cuda")
-    y = torch.empty_like(xd)
-    torch.cuda.synchronize()
-    assert c.L.pf_apply(c.h, PF_FP32_REFINE, C.c_void_p(xd.data_ptr()), C.c_void_p(y.data_ptr())) == 0
-    y = y.cpu().numpy().astype(np.float64).reshape(nz, 2)
+    xd, yd = DeviceArray(x.ravel().astype(np.float32)), DeviceArray(np.zeros(2 * nz, np.float32))
+    assert c.L.pf_apply(c.h, PF_FP32_REFINE, xd.ptr, yd.ptr) == 0
+    y = yd.get().astype(np.float64).reshape(nz, 2)
+    xd.close()
+    yd.close()
     k = np.arange(1, nz - 1)[np.arange(1, nz - 1) % 3 != 0]
     err = np.abs(y[k] / ref[k] - 1.0)
     print("largest error %.3f U" % (err.max() / U), flush=True)
