@@ -378,6 +378,25 @@ def config1(steps, with_cpu):
     return out
 
 
+def batch_level_nodes(n0, n1):
+    """Nodes of an instance's levels outside and inside the kernel of its coarsest levels (the rule
+    of bs_tail_fits: a thread per column and segment of 8 rows, 512 threads, 150 KiB of LDS)."""
+    P = (n1 + 7) // 8
+    W = 1
+    while W < P - 1 and W < 64:
+        W *= 2
+    sizes = [n0]
+    while sizes[-1] > 3:
+        sizes.append(sizes[-1] // 2 + 1)
+    tail = 0
+    for n in sizes[:0:-1]:
+        lds = 6 * (512 + (P if n * W <= 512 else 0))
+        if n * max(P, W) > 512 or n * n1 > lds or 8 * (tail + n * n1 + lds) > 150 * 1024:
+            break
+        tail += n * n1
+    return sum(sizes) * n1 - tail, tail
+
+
 def config3(cpu_seconds):
     """256 uneven 2D cylindrical Shockley instances (plask_amd.workloads.shockley_cyl_batch,
     seeds 3000+i; 50x100 to 400x800 nodes): all instances advancing together, one
@@ -391,7 +410,7 @@ def config3(cpu_seconds):
     nr = np.array([len(p["axes"][0]) for p in insts])
     nz = np.array([len(p["axes"][1]) for p in insts])
     b = ShockleyBatch(insts)
-    blk, nwg, t_tune = b.autotune(maxloops=30)
+    b.solve(want_v=False, maxloops=30)  # tables and graphs
     _, stats, t = b.solve(want_v=False, maxloops=30)
     loops = np.array([s["loops"] for s in stats])
     its = np.array([s["iters"] for s in stats])
@@ -422,21 +441,25 @@ def config3(cpu_seconds):
     work = lambda i: float(nr[i] * nz[i]) * float(nr[i] + 1) ** 2
     c = sum(dt for _, dt in cpu) / sum(work(i) for i, _ in cpu)
     cpu_total = c * sum(loops[i] * work(i) for i in range(len(insts)))
-    # algorithmic bytes (FP64, each value read or written once per pass): per CG iteration
-    # the apply with the direction and solution updates (64 B/node) and the V-cycle, 168 B per
-    # node of every level (first sweep 56, residual 40, way up 72) over levels of 2 N nodes in
-    # all (axis 0 halved per level); per Picard loop the line factors and coarse
-    # conductivities of all levels, the junction update and the currents (~150 B/node)
+    # algorithmic bytes (FP64, each value read or written once per pass): per CG iteration the
+    # apply with the direction and solution updates (64 B/node) and the V-cycle: 156 B per node of
+    # every level outside the tail kernel (first sweep 52, residual 40, way up 64), 72 per node
+    # of those in it (line factors and coefficients read on the way down and up; its vectors stay
+    # in LDS); per Picard loop on all levels the coefficients (32), lines (32), segment factors
+    # (40) and separators (8), on level 0 two true residuals (2 x 32) and the currents (56)
     nodes = (nr * nz).astype(np.float64)
-    bytes_alg = float(np.sum(nodes * (its * (64 + 168 * 2) + loops * 150)))
+    outside, tail = np.array([batch_level_nodes(int(a), int(c)) for a, c in zip(nr, nz)], dtype=np.float64).T
+    bytes_alg = float(np.sum(its * (64 * nodes + 156 * outside + 72 * tail) +
+                             loops * (112 * (outside + tail) + 120 * nodes)))
     roofline = {"bound": "hbm", "kernel": "k_bs_* (whole batch)", "achieved": round(bytes_alg / t / 1e9, 1),
                 "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(bytes_alg / t / 1e9 / HBM_PEAK_GBS, 4),
                 "traffic": None, "bytes": bytes_alg,
-                "note": "late loops hold only the instances that have not converged: their steps are launches of few "
-                        "blocks, held by latency"}
+                "note": "the sweeps fetch about three times their bytes (a block's 40-byte rows of whole lines); late "
+                        "loops hold only the instances that have not converged: launches of few blocks, held by "
+                        "latency"}
     return dict(workload="shockley_cyl_batch_256", instances=len(insts), nodes_total=int((nr * nz).sum()),
                 roofline=roofline,
-                gpu_s=t, block=blk, workgroups=nwg, autotune_s=t_tune, picard_loops_mean=float(loops.mean()),
+                gpu_s=t, picard_loops_mean=float(loops.mean()),
                 picard_loops_max=int(loops.max()), cg_iters_total=int(its.sum()),
                 converged=int((status == 0).sum()), stopped_at_maxloops=int((status == 2).sum()),
                 cpu_sample=[dict(instance=i, seconds_per_loop=dt) for i, dt in cpu],

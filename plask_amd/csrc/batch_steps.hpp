@@ -8,9 +8,9 @@
 // hundreds of dependent rows), and a batch took as long as its slowest instances.  Here the
 // lines are solved by segments (part_solve), the passes of all instances share the chip, and
 // the levels that fit one block's LDS are done in one kernel (k_bs_tail).
-// 24 instances of 20-120 x 40-200 nodes, 6 loops: 130 -> 46 ms (one iteration of all of them is
-// ~15 launches, 190 us, 83 of them the tail).  96 of 50-400 x 100-800, 3 loops: 585 -> 146 ms
-// (1.2 ms an iteration for 9.7e6 nodes on the instance grids).
+// 24 instances of 20-120 x 40-200 nodes, 6 loops: 130 -> 45 ms (one iteration is 11 launches,
+// 190 us, 84 of them the tail).  96 of 50-400 x 100-800, 3 loops: 585 -> 138 ms (23 launches, 1.8 ms
+// an iteration while all of them iterate, 9.7e6 nodes on the instance grids; 1.14 ms on average).
 #pragma once
 #include "batch_kernels.hpp"
 
@@ -18,7 +18,8 @@ namespace pf {
 
 constexpr int BS_M = 8;       // planes per line segment
 constexpr int BS_T = 512;     // threads of a line-sweep block
-constexpr int BS_TAIL = 512;  // threads of a tail block (1024 spill: 95 instead of 49 ms, 24 instances)
+constexpr int BS_TAIL = 512;  // threads of a tail block (256 registers, 20 more spilled; with 1024 threads and 128
+                              // registers most spill: 95 instead of 49 ms, 24 instances)
 
 // One level of one instance (level 0: the instance grid); offsets into the pools of its kind.
 struct BsLevel {
@@ -208,9 +209,11 @@ __device__ __forceinline__ void bs_march(const BsLevel& L, const BsPool& P, int 
 //   k_bs_true     PHASE 0: residual of the start field -> bb; 1: compensated true residual at
 //                 the start of a loop -> its stopping level; 2: after a run -> restart or end
 //                 (march_rows)
-// HBM- (or, on small batches, latency-) bound: 64, 40 and 40 bytes per node; k_bs_apply takes
-// 92 us for 9.7e6 nodes (6.7 TB/s), 10 us for 24 small instances.  Directions are zero at
-// Dirichlet nodes (residuals are), so the elimination only clears the rows there.
+// HBM- (or, on small batches, latency-) bound: 64, 40 and 32 bytes per node; for 9.7e6 nodes
+// k_bs_apply takes 164 us (760 MB moved, 4.6 TB/s), k_bs_resid 102 us (446 MB, 4.4 TB/s),
+// k_bs_true 165 us (its double-double products); 10, 5 and 13 us for 24 small instances.
+// Directions are zero at Dirichlet nodes (residuals are), so the elimination only clears the
+// rows there.
 __global__ __launch_bounds__(256) void k_bs_apply(BsArgs A, const BsBlock* __restrict__ map) {
     const BsBlock B = map[blockIdx.x];
     BsState& S = A.st[B.inst];
@@ -330,7 +333,9 @@ __global__ __launch_bounds__(256) void k_bs_true(BsArgs A, const BsBlock* __rest
 //   UPD    level 0, in an iteration: b -= alpha q (q in r, overwritten) before it, (b, b) and
 //          the stop test
 //   DOWN   coarse level: b = R r of the finer level's residual (stored)
-// 56 bytes per node; UPD 122 us for 9.7e6 nodes (4.4 TB/s), 11 us for 24 small instances.
+// 36, 52 and 52 bytes per node, 4 of them of the separators.  UPD 223 us for 9.7e6 nodes, 10 us for
+// 24 small instances.  What holds it on large ones is HBM, at 2.7 times those bytes (1380 MB, 6.2
+// TB/s): a block reads L.CB columns of a row, 5 (40 bytes) at 800 rows, and fetches whole lines.
 enum { BS_START = 0, BS_UPD = 1, BS_DOWN = 2 };
 
 template <int MODE>
@@ -485,8 +490,10 @@ __device__ __forceinline__ void bs_lds_residual(const BsLevel& L, const double* 
 // each side in LDS, then x = x' + omega M^-1 (b - A x') (on level 0 also (b, x) and the next
 // beta).  x is read from r (where the way down left it, see steps_vcycle) and written to x, as
 // neighbouring blocks read the columns around theirs.  As three kernels (correction, residual,
-// sweep) it moved 108 instead of 72 bytes per node and cost three launches: 157 -> 146 ms for
-// 96 uneven instances, 49 -> 46 ms for 24 small ones.  x' is staged rather than read around each
+// sweep) it needs 104 instead of 64 bytes per node and three launches: 157 -> 146 ms for
+// 96 uneven instances, 49 -> 46 ms for 24 small ones.  358 us for the 9.7e6 nodes of the instance
+// grids, held by HBM at 3.4 times those bytes (2100 MB, 5.9 TB/s): the narrow rows of the sweeps,
+// and two columns more per block.  x' is staged rather than read around each
 // thread because the columns of a segment are M rows apart; the pad per segment puts the
 // segments of a column into different banks.
 __host__ __device__ inline int bs_up_pad(int CB) { return ((CB - BS_M * (CB + 2)) % 32 + 32) % 32; }

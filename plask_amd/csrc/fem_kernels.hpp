@@ -1566,8 +1566,8 @@ __host__ __device__ inline int part_lds_values(int P, int CB, int S) {
 // A vector's values of a thread's segment, 0 past its end.  No branch per value (each would wait
 // for the kernel arguments of its address anew): threads and planes past the end read the
 // segment's first plane, or node 0, and drop it.  Long segments skip the selects where a wave
-// holds whole ones (16 planes FP32, 96 x 96 x 192 nodes: 15.0 us with them, 12.6 without, 13.4
-// with branches; 4 planes FP64, 25 x 19 x 37 nodes: 4.3 us, with branches 4.6; 8 planes with the
+// holds whole ones (16 planes FP32, 96 x 96 x 192 nodes, with c' formed from a and w: 15.0 us with
+// them, 12.6 without, 13.4 with branches; 14.5 without them now that c' is read; 4 planes FP64, 25 x 19 x 37 nodes: 4.3 us, with branches 4.6; 8 planes with the
 // residual update, 128 x 128 x 256: 42 us, with branches 47.6).
 template <typename T, int M>
 __device__ __forceinline__ void part_load(const PartPos& q, long long plane, const T* __restrict__ v, T (&out)[M]) {

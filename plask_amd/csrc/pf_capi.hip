@@ -1763,9 +1763,10 @@ static void mg_vcycle(pf_ctx* ctx, T* r, const T* q, T* z, bool upd, int fin) {
     const int L = (int)ctx->mg.size() + 1;
     const bool fuse = ctx->mg_fuse && ctx->dim == 3 && L > 1 && ctx->apply_kind[sizeof(T) == 8 ? 0 : 1] == 0;
     // restriction inside the level's first sweep: everywhere with fused transfers, and otherwise
-    // in FP64 on the 3D levels of 4-plane segments (at most 512 columns), where a launch costs more
-    // than the sweep's gather (2.7 us against 0.4 per level: 25 x 19 x 37 nodes 1.76 -> 1.70 ms,
-    // 97 x 83 x 131 3.93 -> 3.90; FP32, 96 x 96 x 192: 3.88 -> 3.91, so not there)
+    // in FP64 on the 3D levels of 4-plane segments (at most 512 columns), where a launch of about 3 us
+    // costs more than the sweep's gather (0.3-0.4 us per level at 25 x 19 x 37 nodes, 1.70 instead of
+    // 1.76 ms; at 97 x 83 x 131 3.90 instead of 3.93 ms; 1.7-3.5 us per level at 128 x 128 x 256;
+    // FP32, 96 x 96 x 192: 3.91 instead of 3.88 ms, so not there)
     auto restricts = [&](const MgView<T>& v) {
         return fuse || (sizeof(T) == 8 && ctx->dim == 3 && part_shape<T>(v.pm, v.planes, v.ncol).m == 4);
     };
